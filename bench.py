@@ -526,12 +526,13 @@ def main():
     err_fp64 = float(np.linalg.norm(x_fp64 - x_ref) / np.linalg.norm(x_ref))
 
     # ---- roofline of the dominant kernel: level-0 FP32 smoother ----
-    # Algorithmic bytes per point of a GS update: 27 coefficients + r + x
-    # read + x write = 30 words; FP32 = 120 B.  One forward launch updates
-    # two colour classes, N0/4 points on average; the timing hook counts the
+    # Algorithmic bytes per point of a GS update on this operator, a 7-point
+    # cross: 7 coefficients + r + x read + x write = 10 words (the 20 planes
+    # of zeros are not read); FP32 = 40 B.  One forward launch updates two
+    # colour classes, N0/4 points on average; the timing hook counts the
     # points exactly.
     avg_launch_s = (ms_gs / 1000.0) / max(n_gs, 1)
-    bytes_launch = 120.0 * pts_gs / max(n_gs, 1)
+    bytes_launch = 40.0 * pts_gs / max(n_gs, 1)
     achieved = bytes_launch / avg_launch_s / 1e9
     traffic = None
     tf = os.path.join(ROOT, "profiles", "traffic_gs_pair_f32_257.json")
@@ -574,7 +575,7 @@ def main():
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic, "launches": n_gs, "avg_launch_us": round(1e6 * avg_launch_s, 2),
                      "bytes_per_launch": bytes_launch},
-        "roofline_fp64_gs": {"achieved": round(240.0 * pts_gs64 / (ms_gs64 / 1000.0) / 1e9, 1),
+        "roofline_fp64_gs": {"achieved": round(80.0 * pts_gs64 / (ms_gs64 / 1000.0) / 1e9, 1),
                              "avg_launch_us": round(1000.0 * ms_gs64 / max(n_gs64, 1), 2)},
         "roofline_exact": roofline_exact,
     }

@@ -83,8 +83,10 @@ struct pgmg_hier {
 	double *partial = nullptr;
 	int partial_cap = 0;
 	double *dscalar = nullptr;  // device reduction result; the int after it is the
-	                            // exact sweeps' wait flag (set when a wait gave up)
-	double *hscalar = nullptr;  // pinned host mirror of both
+	                            // exact sweeps' wait flag (set when a wait gave up),
+	                            // the int in the third double the upload's
+	                            // dense-operator flag
+	double *hscalar = nullptr;  // pinned host mirror of the three
 	int *flow_prog = nullptr;   // plane progress counters of the exact sweeps
 	int flow_limit = kFlowLimit;
 	double *LU = nullptr;
@@ -607,9 +609,9 @@ int pgmg_hier_create(const pgmg_dims *d, const pgmg_opts *opts, pgmg_hier **out)
 		ALLOC(h->res32, np0 * 4);
 		launch_fill<float>(h->stream, h->res32, (long long)np0, 0.0f);
 	}
-	ALLOC(h->dscalar, 16);
-	launch_fill<double>(h->stream, h->dscalar, 2, 0.0);
-	if (hipHostMalloc((void **)&h->hscalar, 16) != hipSuccess) { pgmg_hier_destroy(h); return fail(PGMG_ERR_MEMORY, "pinned alloc failed"); }
+	ALLOC(h->dscalar, 24);
+	launch_fill<double>(h->stream, h->dscalar, 3, 0.0);
+	if (hipHostMalloc((void **)&h->hscalar, 24) != hipSuccess) { pgmg_hier_destroy(h); return fail(PGMG_ERR_MEMORY, "pinned alloc failed"); }
 	rc = ensure_partial(h, residual_partial_count(h->lev[0].v));
 	if (rc) { pgmg_hier_destroy(h); return rc; }
 #undef ALLOC
@@ -651,29 +653,40 @@ int pgmg_level_dims(const pgmg_hier *h, int level, int dims[3]) {
 	return PGMG_OK;
 }
 
-static int upload_op(pgmg_hier *h, int level, const double *A27) {
-	Level &L = h->lev[level];
+// Host operator into level 0, and whether it is a 7-point cross (its 20 other
+// entries zero at every point), which the smoother and residual kernels use.
+static int upload_op(pgmg_hier *h, const double *A27) {
+	Level &L = h->lev[0];
 	const long long N = L.points();
 	const long long chunk = 1 << 20;
 	double *stage = nullptr;
+	int *dense = (int *)(h->dscalar + 2);
 	HIP_TRY(hipMalloc(&stage, sizeof(double) * 27 * (size_t)std::min(N, chunk)));
+	// from here on the level holds neither operator: read every entry
+	L.v.cross = 0;
+	free_graphs(h);
+	launch_fill<int>(h->stream, dense, 1, 0);
 	for (long long p0 = 0; p0 < N; p0 += chunk) {
 		const long long cnt = std::min(chunk, N - p0);
 		hipError_t e = hipMemcpyAsync(stage, A27 + 27 * p0, sizeof(double) * 27 * cnt, hipMemcpyHostToDevice, h->stream);
 		if (e != hipSuccess) { hipFree(stage); return fail(PGMG_ERR_HIP, "upload: %s", hipGetErrorString(e)); }
-		launch_pack_op(h->stream, L.v, stage, L.A, p0, cnt);
+		launch_pack_op(h->stream, L.v, stage, L.A, p0, cnt, dense);
 		hipStreamSynchronize(h->stream);
 	}
 	hipFree(stage);
+	HIP_TRY(hipMemcpyAsync(h->hscalar + 2, h->dscalar + 2, sizeof(double), hipMemcpyDeviceToHost, h->stream));
+	HIP_TRY(hipStreamSynchronize(h->stream));
+	int d = 1;
+	memcpy(&d, h->hscalar + 2, sizeof(int));
+	L.v.cross = d == 0 && cross_pays(L.v);
 	return PGMG_OK;
 }
 
 int pgmg_set_operator27(pgmg_hier *h, const double *A27) {
 	if (!h || !A27) return fail(PGMG_ERR_ARG, "null argument");
-	int rc = upload_op(h, 0, A27);
+	int rc = upload_op(h, A27);
 	if (rc) return rc;
 	h->ops_ready = false;
-	free_graphs(h);
 	return PGMG_OK;
 }
 
@@ -681,6 +694,7 @@ int pgmg_generate_problem(pgmg_hier *h, int family, uint64_t seed) {
 	if (!h) return fail(PGMG_ERR_ARG, "null hierarchy");
 	if (family != PGMG_FAM_FACE7_UNIFORM && family != PGMG_FAM_FACE7_LOGUNI && family != PGMG_FAM_Q1_ANISO)
 		return fail(PGMG_ERR_ARG, "unknown problem family %d", family);
+	h->lev[0].v.cross = family != PGMG_FAM_Q1_ANISO && cross_pays(h->lev[0].v);
 	launch_generate(h->stream, h->lev[0].v, family, seed, h->lev[0].A, h->lev[0].r);
 	HIP_TRY(hipStreamSynchronize(h->stream));
 	h->ops_ready = false;

@@ -30,11 +30,25 @@ struct LevelView {
 	long long pxy;     // plane pitch (elements)
 	long long base;    // index of point (0,0,0)
 	long long npad;    // elements per array, halo included
-	int cache_coef;    // 1: levels run one at a time (a lone hierarchy), so a
+	short cache_coef;  // 1: levels run one at a time (a lone hierarchy), so a
 	                   // level may keep coefficients in the memory-side cache;
 	                   // 0: stream them (batched slots run side by side)
+	short cross;       // 1: every coefficient outside the 7-point cross is
+	                   // zero (see in_cross); the kernels do not read them
 	int prd;           // periodic axes: bit 0 x, bit 1 y, bit 2 z
 };
+
+// Entries of the 7-point cross: the centre and its six face neighbours.
+__host__ __device__ constexpr bool in_cross(int e) {
+	return e == 4 || e == 10 || e == 12 || e == 13 || e == 14 || e == 16 || e == 22;
+}
+
+// Whether a level whose operator is a 7-point cross is worth the kernels that
+// read 7 planes (40 instead of 120 bytes a point in FP32).  Small levels are
+// bound by the latency of a launch, not by bytes: mixed solves, 33^3 (36 k
+// points) 2.69 ms with the cross kernels and 2.67 without, 65^3 (275 k) 4.22
+// and 4.27, 129^3 7.08 and 8.94, 257^3 23.3 and 39.0.
+inline bool cross_pays(const LevelView &v) { return (long long)v.m * v.n * v.o >= 65536; }
 
 inline LevelView make_level_view(int m, int n, int o) {
 	LevelView v;
@@ -47,6 +61,7 @@ inline LevelView make_level_view(int m, int n, int o) {
 	v.npad = v.pxy * (o + 2);
 	v.cache_coef = 0;
 	v.prd = 0;
+	v.cross = 0;
 	return v;
 }
 
@@ -325,7 +340,10 @@ void launch_generate(hipStream_t s, const LevelView &L, int family, uint64_t see
 // and the padded level layout, for points [p0, p0+count).
 void launch_pack_vec(hipStream_t s, const LevelView &L, const double *compact, double *padded, long long p0, long long count);
 void launch_unpack_vec(hipStream_t s, const LevelView &L, const double *padded, double *compact, long long p0, long long count);
-void launch_pack_op(hipStream_t s, const LevelView &L, const double *compact27, double *A, long long p0, long long count);
+// launch_pack_op sets *dense to 1 when an entry outside the 7-point cross is
+// not zero, and leaves it otherwise.
+void launch_pack_op(hipStream_t s, const LevelView &L, const double *compact27, double *A, long long p0, long long count,
+		    int *dense = nullptr);
 void launch_unpack_op(hipStream_t s, const LevelView &L, const double *A, double *compact27, long long p0, long long count);
 // Elementwise helpers.
 template <typename T> void launch_fill(hipStream_t s, T *p, long long n, T v);

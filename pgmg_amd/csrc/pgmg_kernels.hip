@@ -32,7 +32,10 @@ __device__ __forceinline__ int xcd_block(int b, int G) {
 // Gauss-Seidel update of point (i,j,k) (region.cc:369-438): sum over the
 // 26 off-centre entries in box order from zero, then
 // x = (r - Ax) * (1/a_centre) with the reciprocal taken first.
-template <typename T>
+// X: the level's operator is a 7-point cross (LevelView::cross), whose other
+// coefficients are taken as 0 instead of read (in the row kernels too; see
+// coef_or_zero).
+template <typename T, bool X = false>
 __device__ __forceinline__ void gs_point(const LevelView &L, const T *__restrict__ A, T *__restrict__ x,
 					 const T *__restrict__ r, int i, int j, int k) {
 	const long long px = L.px, pxy = L.pxy, p = idx3(L, i, j, k);
@@ -42,7 +45,8 @@ __device__ __forceinline__ void gs_point(const LevelView &L, const T *__restrict
 	for (int e = 0; e < 27; e++) {
 		if (e == 13) continue;
 		const int di = e % 3 - 1, dj = (e / 3) % 3 - 1, dk = e / 9 - 1;
-		ax = ax + Ap[e * L.pa] * x[p + di + dj * px + dk * pxy];
+		const T a = X && !in_cross(e) ? (T)0 : Ap[e * L.pa];
+		ax = ax + a * x[p + di + dj * px + dk * pxy];
 	}
 	x[p] = (r[p] - ax) * ((T)1 / Ap[13 * L.pa]);
 }
@@ -120,14 +124,14 @@ void launch_halo_wrap(hipStream_t s, const LevelView &L, T *x) {
 
 // One colour class: points (2a+ci, 2b+cj, 2d+ck).  Points of one class never
 // share a stencil box, so all of them update in parallel.
-template <typename T>
+template <typename T, bool X>
 __global__ __launch_bounds__(256) void k_gs_colour(LevelView L, const T *__restrict__ A, T *__restrict__ x,
 						   const T *__restrict__ r, int ci, int cj, int ck) {
 	const int i = 2 * (int)(blockIdx.x * 64 + threadIdx.x) + ci;
 	const int j = 2 * (int)(blockIdx.y * 4 + threadIdx.y) + cj;
 	const int k = 2 * (int)blockIdx.z + ck;
 	if (i >= L.m || j >= L.n || k >= L.o) return;
-	gs_point<T>(L, A, x, r, i, j, k);
+	gs_point<T, X>(L, A, x, r, i, j, k);
 }
 
 template <typename T>
@@ -136,7 +140,8 @@ void launch_gs_colour(hipStream_t s, const LevelView &L, const T *A, T *x, const
 	const int na = (L.m - ci + 1) / 2, nb = (L.n - cj + 1) / 2, nd = (L.o - ck + 1) / 2;
 	if (na <= 0 || nb <= 0 || nd <= 0) return;
 	dim3 grid((na + 63) / 64, (nb + 3) / 4, nd), block(64, 4, 1);
-	hipLaunchKernelGGL(k_gs_colour<T>, grid, block, 0, s, L, A, x, r, ci, cj, ck);
+	if (L.cross) hipLaunchKernelGGL((k_gs_colour<T, true>), grid, block, 0, s, L, A, x, r, ci, cj, ck);
+	else hipLaunchKernelGGL((k_gs_colour<T, false>), grid, block, 0, s, L, A, x, r, ci, cj, ck);
 	HIPCHECK_LAUNCH();
 }
 
@@ -197,6 +202,27 @@ template <> __device__ __forceinline__ double2 ld_stream<double2>(const void *ba
 	return make_double2(v.x, v.y);
 }
 
+// The vector of coefficient plane e at byte offset off of row block Ar, or,
+// on a level whose operator is a 7-point cross (X), a zero for the 20 planes
+// outside the cross, which are not read.  The caller keeps their terms
+// (0 * x), so the sums are those of the 27 planes for every x, infinities and
+// NaN included; e must be a compile-time constant after unrolling.  The row
+// kernels are bound by HBM bytes, and 20 of the 27 planes of a 7-point
+// operator hold only zeros: 257^3 level-0 smoother launch FP32 98 -> 42 us
+// (5.3 TB/s of the 13 words a point it then moves), FP64 210 -> 101 us; FP64
+// residual 666 -> 301 us.
+template <typename V, bool X, typename T>
+__device__ __forceinline__ V coef_or_zero(const T *Ar, int e, long long pa, uint32_t off) {
+	if (X && !in_cross(e)) {
+		V z;
+		T *pz = reinterpret_cast<T *>(&z);
+#pragma unroll
+		for (int t = 0; t < (int)(sizeof(V) / sizeof(T)); t++) pz[t] = (T)0;
+		return z;
+	}
+	return ld_stream<V>(Ar + e * pa, off);
+}
+
 // First sweep from x = 0 (template flag Z of the FP32 row kernels): the rows of this colour pair and of the pairs
 // after it have not been updated yet in the sweep, so they still hold 0;
 // their x is not read (the caller need not clear x), and the terms see the
@@ -252,7 +278,7 @@ __device__ __forceinline__ T read_lane(T v, int l) {
 }
 // ALL: every lane forms the point out's sum, with no branch (see below); the
 // batched kernel keeps it in lane 63's branch, which holds it to 256 VGPRs.
-template <typename T, bool ALL = true>
+template <typename T, bool ALL = true, bool X = false>
 __device__ __forceinline__ void gs_pair_row(const LevelView &L, const T *__restrict__ A, T *__restrict__ x,
 					    const T *__restrict__ r, int j, int k) {
 	typedef typename Vec2<T>::type V2;
@@ -303,9 +329,9 @@ __device__ __forceinline__ void gs_pair_row(const LevelView &L, const T *__restr
 			for (int rq = 0; rq < 9; rq++) {
 				const int dj = rq % 3 - 1, dk = rq / 3 - 1;
 				const T *xq = xr + dj * px + dk * pxy;
-				const V2 am = ld_stream<V2>(Ar + (3 * rq) * pa, ob);
-				const V2 a0 = ld_stream<V2>(Ar + (3 * rq + 1) * pa, ob);
-				const V2 ap = ld_stream<V2>(Ar + (3 * rq + 2) * pa, ob);
+				const V2 am = coef_or_zero<V2, X>(Ar, 3 * rq, pa, ob);
+				const V2 a0 = coef_or_zero<V2, X>(Ar, 3 * rq + 1, pa, ob);
+				const V2 ap = coef_or_zero<V2, X>(Ar, 3 * rq + 2, pa, ob);
 				const V2 xv = ld_row<V2>(xq, ob);
 				const T xm = ld_row<T>(xq - 1, ob);
 				const T xp = doO ? ld_row<T>(xq + 2, ob) : (T)0;
@@ -389,7 +415,7 @@ __device__ __forceinline__ void gs_pair_row(const LevelView &L, const T *__restr
 // stores are issued after the next segment's loads, as in gs_pair_row.
 // Per-point arithmetic and order as in gs_point.  j and k must be
 // wavefront-uniform.
-template <bool Z = false>
+template <bool Z = false, bool X = false>
 __device__ __forceinline__ void gs_quad_row_f32(const LevelView &L, const float *__restrict__ A, float *__restrict__ x,
 						const float *__restrict__ r, int j, int k) {
 	const int cj = j & 1, ck = k & 1;
@@ -444,9 +470,9 @@ __device__ __forceinline__ void gs_quad_row_f32(const LevelView &L, const float 
 			for (int rq = 0; rq < 9; rq++) {
 				const int dj = rq % 3 - 1, dk = rq / 3 - 1;
 				const float *xq = xr + dj * px + dk * pxy;
-				const float4 am = ld_stream<float4>(Ar + (3 * rq) * pa, ob);
-				const float4 a0 = ld_stream<float4>(Ar + (3 * rq + 1) * pa, ob);
-				const float4 ap = ld_stream<float4>(Ar + (3 * rq + 2) * pa, ob);
+				const float4 am = coef_or_zero<float4, X>(Ar, 3 * rq, pa, ob);
+				const float4 a0 = coef_or_zero<float4, X>(Ar, 3 * rq + 1, pa, ob);
+				const float4 ap = coef_or_zero<float4, X>(Ar, 3 * rq + 2, pa, ob);
 				const bool zr = Z && zero_row(cj, ck, dj, dk);
 				float4 xv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 				float xm = 0.0f, xp = 0.0f;
@@ -571,11 +597,15 @@ __device__ __forceinline__ void ld_vec_stream(const T *base, uint32_t off, T (&o
 // one (two cost level 1 its cached planes).  Batched slots run side by side,
 // their levels together far larger than the cache: they stream everything
 // (measured: 256-problem batch 16.3 s with the per-level rule, 13.6 s
-// streamed).
-template <typename T>
+// streamed).  A 7-point cross (X) reads 7 planes, 4, 10, 12, 13, 14, 16 and
+// 22: all kept where they fit, else one plane as above (split 5 keeps plane
+// 4).  257^3 mixed solve 23.5 ms streamed, 23.3 with one plane, 23.3 with two,
+// 23.4 with four; FP64 38.5 ms in every case.
+template <typename T, bool X>
 __device__ __forceinline__ int coef_split(const LevelView &L) {
 	if (!L.cache_coef) return 0;
 	const long long plane = (long long)L.m * L.n * L.o * (long long)sizeof(T);
+	if (X) return 7 * plane <= (256LL << 20) ? 27 : plane <= (80LL << 20) ? 5 : 0;
 	if (27 * plane <= (256LL << 20)) return 27;
 	if (27 * plane <= (1024LL << 20)) return 9;
 	return plane <= (80LL << 20) ? 1 : 0;
@@ -584,6 +614,16 @@ template <typename T, int N>
 __device__ __forceinline__ void ld_vec_coef(const T *base, uint32_t off, T (&out)[N], bool nt) {
 	if (nt) ld_vec_stream<T, N>(base, off, out);
 	else ld_vec<T, N>(base, off, out);
+}
+// Coefficient plane e in the packed-row kernels; X as in coef_or_zero.
+template <typename T, int N, bool X>
+__device__ __forceinline__ void ld_coef_lanes(const T *Ab, int e, long long pa, uint32_t off, T (&out)[N], int split) {
+	if (X && !in_cross(e)) {
+#pragma unroll
+		for (int t = 0; t < N; t++) out[t] = (T)0;
+		return;
+	}
+	ld_vec_coef<T, N>(Ab + e * pa, off, out, e >= split);
 }
 template <typename T, int N>
 __device__ __forceinline__ void st_vec(T *base, uint32_t off, const T (&v)[N]) {
@@ -615,7 +655,7 @@ enum { PO_NONE = 0, PO_ROWS = 1, PO_TAIL = 2 };
 // planes are reached; plain loads, so a level that keeps its coefficients
 // cached keeps the copy cached too.  rq must be a compile-time constant (an
 // unrolled loop), so tb stays in registers.
-template <typename T>
+template <typename T, bool X>
 __device__ __forceinline__ void point_out_tail(const T *Ab, uint32_t ot, int rq, T (&tb)[28], T (&b)[3]) {
 	constexpr int VW = 16 / (int)sizeof(T);
 #pragma unroll
@@ -627,7 +667,7 @@ __device__ __forceinline__ void point_out_tail(const T *Ab, uint32_t ot, int rq,
 #pragma unroll
 			for (int q = 0; q < VW; q++) tb[e + q] = v[q];
 		}
-		b[d] = tb[e];
+		b[d] = X && !in_cross(e) ? (T)0 : tb[e];
 	}
 }
 
@@ -641,7 +681,7 @@ __device__ __forceinline__ void point_out_tail(const T *Ab, uint32_t ot, int rq,
 // at a row's last lane the point out (or the halo).  Only the wavefront's
 // rows are written by the launch, so each lane stores its points once, at
 // the end.  Per-point arithmetic and order as in gs_point.
-template <typename T, int PPL, bool Z, int PO>
+template <typename T, int PPL, bool Z, int PO, bool X = false>
 __device__ __forceinline__ void gs_lanes(const LevelView &L, const T *__restrict__ A, T *__restrict__ x,
 					 const T *__restrict__ r, int cj, int ck, int q0, int nrows) {
 	const RowLanes W = row_lanes(L.m, (int)sizeof(T));
@@ -653,7 +693,7 @@ __device__ __forceinline__ void gs_lanes(const LevelView &L, const T *__restrict
 	const int j0 = 2 * (q0 % nb) + cj, k0 = 2 * (q0 / nb) + ck;
 	const long long xb0 = idx3(L, 0, j0, k0), ab0 = arow0(L, j0, k0);
 	const long long px = L.px, pxy = L.pxy, pa = L.pa;
-	const int split = coef_split<T>(L);
+	const int split = coef_split<T, X>(L);
 	const T *Ab = A + ab0;
 	const T *rb = r + xb0;
 	T *xb = x + xb0;
@@ -685,7 +725,7 @@ __device__ __forceinline__ void gs_lanes(const LevelView &L, const T *__restrict
 			const T *xq = xb + dj * px + dk * pxy;
 			T a[3][PPL], xv[PPL];
 #pragma unroll
-			for (int d = 0; d < 3; d++) ld_vec_coef<T, PPL>(Ab + (3 * rq + d) * pa, oa, a[d], 3 * rq + d >= split);
+			for (int d = 0; d < 3; d++) ld_coef_lanes<T, PPL, X>(Ab, 3 * rq + d, pa, oa, a[d], split);
 			T xm = (T)0, xp = (T)0;
 			if (Z && zero_row(cj, ck, dj, dk)) {
 #pragma unroll
@@ -697,11 +737,12 @@ __device__ __forceinline__ void gs_lanes(const LevelView &L, const T *__restrict
 			}
 			T b[3] = {(T)0, (T)0, (T)0};
 			if constexpr (PO == PO_TAIL) {
-				point_out_tail<T>(Ab, ot, rq, tb, b);
+				point_out_tail<T, X>(Ab, ot, rq, tb, b);
 			} else if constexpr (PO == PO_ROWS) {
 				if (ext) {
 #pragma unroll
-					for (int d = 0; d < 3; d++) b[d] = ld_row<T>(Ab + (3 * rq + d) * pa, oa + oe);
+					for (int d = 0; d < 3; d++)
+						if (!X || in_cross(3 * rq + d)) b[d] = ld_row<T>(Ab + (3 * rq + d) * pa, oa + oe);
 				}
 			}
 			if (rq == 4) {
@@ -791,7 +832,7 @@ __device__ __forceinline__ void gs_lanes(const LevelView &L, const T *__restrict
 // Residual of rows that fit one wavefront's lanes (layout as gs_lanes);
 // returns this lane's sum of squares.  zx (may be null) is set to 0 at the
 // same points.
-template <typename T, typename TR, int PPL, int PO>
+template <typename T, typename TR, int PPL, int PO, bool X = false>
 __device__ __forceinline__ double residual_lanes(const LevelView &L, const T *__restrict__ A, const T *__restrict__ x,
 						 const T *__restrict__ r, TR *__restrict__ res, TR *__restrict__ zx,
 						 int q0, int nrows) {
@@ -803,7 +844,7 @@ __device__ __forceinline__ double residual_lanes(const LevelView &L, const T *__
 	const int j0 = q0 % L.n, k0 = q0 / L.n;
 	const long long xb0 = idx3(L, 0, j0, k0), ab0 = arow0(L, j0, k0);
 	const long long px = L.px, pxy = L.pxy, pa = L.pa;
-	const int split = coef_split<T>(L);
+	const int split = coef_split<T, X>(L);
 	double v2 = 0.0;
 	if (!live) return v2;
 	const int j = q % L.n, k = q / L.n;
@@ -830,7 +871,7 @@ __device__ __forceinline__ double residual_lanes(const LevelView &L, const T *__
 		const T *xq = xb + dj * px + dk * pxy;
 		T a[3][PPL], xv[PPL];
 #pragma unroll
-		for (int d = 0; d < 3; d++) ld_vec_coef<T, PPL>(Ab + (3 * rq + d) * pa, oa, a[d], 3 * rq + d >= split);
+		for (int d = 0; d < 3; d++) ld_coef_lanes<T, PPL, X>(Ab, 3 * rq + d, pa, oa, a[d], split);
 		ld_vec<T, PPL>(xq, ox, xv);
 		const T xm = ld_row<T>(xq - 1, ox);
 		const T xp = needxp ? ld_row<T>(xq + PPL, ox) : (T)0;
@@ -844,7 +885,7 @@ __device__ __forceinline__ double residual_lanes(const LevelView &L, const T *__
 		}
 		if constexpr (PO == PO_TAIL) {
 			T b[3];
-			point_out_tail<T>(Ab, ot, rq, tb, b);
+			point_out_tail<T, X>(Ab, ot, rq, tb, b);
 			// every lane sums; only the last lane's sx is used
 			sx = sx + b[0] * xv[PPL - 1];
 			sx = sx + b[1] * xp;
@@ -854,9 +895,13 @@ __device__ __forceinline__ double residual_lanes(const LevelView &L, const T *__
 			// share the addresses) and sums, with no branch; only the last
 			// lane's sx is used
 			if (W.ext) {
-				sx = sx + ld_row<T>(Ab + (3 * rq) * pa, oz) * xv[PPL - 1];
-				sx = sx + ld_row<T>(Ab + (3 * rq + 1) * pa, oz) * xp;
-				sx = sx + ld_row<T>(Ab + (3 * rq + 2) * pa, oz) * (T)0;  // the halo point i = m
+				T b[3];
+#pragma unroll
+				for (int d = 0; d < 3; d++)
+					b[d] = X && !in_cross(3 * rq + d) ? (T)0 : ld_row<T>(Ab + (3 * rq + d) * pa, oz);
+				sx = sx + b[0] * xv[PPL - 1];
+				sx = sx + b[1] * xp;
+				sx = sx + b[2] * (T)0;  // the halo point i = m
 			}
 		}
 	}
@@ -895,14 +940,14 @@ __device__ __forceinline__ double residual_lanes(const LevelView &L, const T *__
 // two in FP64 (whose 16-byte pair loads already fill the registers).
 // The first-sweep-from-zero form (Z) exists in FP32 only.  ALL: as in
 // gs_pair_row.
-template <typename T, bool Z, bool ALL = true>
+template <typename T, bool Z, bool ALL = true, bool X = false>
 __device__ __forceinline__ void gs_row(const LevelView &L, const T *__restrict__ A, T *__restrict__ x,
 				       const T *__restrict__ r, int j, int k) {
 	if constexpr (sizeof(T) == 4) {
-		gs_quad_row_f32<Z>(L, A, x, r, j, k);
+		gs_quad_row_f32<Z, X>(L, A, x, r, j, k);
 	} else {
 		static_assert(!Z, "first sweep from zero: FP32 only");
-		gs_pair_row<T, ALL>(L, A, x, r, j, k);
+		gs_pair_row<T, ALL, X>(L, A, x, r, j, k);
 	}
 }
 
@@ -911,7 +956,7 @@ template <typename T> struct Ppl { static const int v = sizeof(T) == 4 ? 4 : 2; 
 // Wavefront w of a colour-pair launch: rows w*rpw .. of the pair when they
 // fit the lanes, else the single long row w, streamed in segments.  w must be
 // wavefront-uniform.
-template <typename T, bool Z = false, bool ALL = true>
+template <typename T, bool Z = false, bool ALL = true, bool X = false>
 __device__ __forceinline__ void gs_wave(const LevelView &L, const T *__restrict__ A, T *__restrict__ x,
 					const T *__restrict__ r, int cj, int ck, int w) {
 	const int nb = (L.n - cj + 1) >> 1, nd = (L.o - ck + 1) >> 1, rows = nb * nd;
@@ -920,20 +965,20 @@ __device__ __forceinline__ void gs_wave(const LevelView &L, const T *__restrict_
 		const int q0 = w * W.rpw;
 		if (q0 < rows) {
 			// FP32 point outs come with a tail copy (m = 4q+1)
-			if constexpr (sizeof(T) == 8) gs_lanes<T, Ppl<T>::v, Z, PO_ROWS>(L, A, x, r, cj, ck, q0, rows);
-			else if (W.ext) gs_lanes<T, Ppl<T>::v, Z, PO_TAIL>(L, A, x, r, cj, ck, q0, rows);
-			else gs_lanes<T, Ppl<T>::v, Z, PO_NONE>(L, A, x, r, cj, ck, q0, rows);
+			if constexpr (sizeof(T) == 8) gs_lanes<T, Ppl<T>::v, Z, PO_ROWS, X>(L, A, x, r, cj, ck, q0, rows);
+			else if (W.ext) gs_lanes<T, Ppl<T>::v, Z, PO_TAIL, X>(L, A, x, r, cj, ck, q0, rows);
+			else gs_lanes<T, Ppl<T>::v, Z, PO_NONE, X>(L, A, x, r, cj, ck, q0, rows);
 		}
 	} else if (w < rows) {
-		gs_row<T, Z, ALL>(L, A, x, r, 2 * (w % nb) + cj, 2 * (w / nb) + ck);
+		gs_row<T, Z, ALL, X>(L, A, x, r, 2 * (w % nb) + cj, 2 * (w / nb) + ck);
 	}
 }
 
-template <typename T, bool Z = false>
+template <typename T, bool Z, bool X>
 __global__ __launch_bounds__(256) void k_gs_pair(LevelView L, const T *__restrict__ A, T *__restrict__ x,
 						 const T *__restrict__ r, int cj, int ck) {
 	const int w = __builtin_amdgcn_readfirstlane(xcd_block((int)blockIdx.x, (int)gridDim.x) * (int)blockDim.y + (int)threadIdx.y);
-	gs_wave<T, Z>(L, A, x, r, cj, ck, w);
+	gs_wave<T, Z, true, X>(L, A, x, r, cj, ck, w);
 }
 
 // Wavefronts of one colour-pair launch.
@@ -957,12 +1002,14 @@ void launch_gs_pair(hipStream_t s, const LevelView &L, const T *A, T *x, const T
 	const dim3 grid((waves + kGsRows - 1) / kGsRows), block(64, kGsRows, 1);
 	if constexpr (sizeof(T) == 4) {
 		if (from_zero) {
-			hipLaunchKernelGGL((k_gs_pair<T, true>), grid, block, 0, s, L, A, x, r, cj, ck);
+			if (L.cross) hipLaunchKernelGGL((k_gs_pair<T, true, true>), grid, block, 0, s, L, A, x, r, cj, ck);
+			else hipLaunchKernelGGL((k_gs_pair<T, true, false>), grid, block, 0, s, L, A, x, r, cj, ck);
 			HIPCHECK_LAUNCH();
 			return;
 		}
 	}
-	hipLaunchKernelGGL((k_gs_pair<T, false>), grid, block, 0, s, L, A, x, r, cj, ck);
+	if (L.cross) hipLaunchKernelGGL((k_gs_pair<T, false, true>), grid, block, 0, s, L, A, x, r, cj, ck);
+	else hipLaunchKernelGGL((k_gs_pair<T, false, false>), grid, block, 0, s, L, A, x, r, cj, ck);
 	HIPCHECK_LAUNCH();
 }
 
@@ -1797,7 +1844,7 @@ __device__ __forceinline__ double block_sum_256(double v) {
 // blocks of 4 wavefronts, renumbered per XCD.
 // res (may be null) receives the residual in type TR, partial (may be null)
 // one sum per block.  q and seg must be wavefront-uniform.
-template <typename T, typename TR>
+template <typename T, typename TR, bool X>
 __device__ __forceinline__ double residual_row_pair(const LevelView &L, const T *__restrict__ A, const T *__restrict__ x,
 						    const T *__restrict__ r, TR *__restrict__ res, int q, int seg,
 						    TR *__restrict__ zx = nullptr) {
@@ -1854,9 +1901,9 @@ __device__ __forceinline__ double residual_row_pair(const LevelView &L, const T 
 				for (int rq = 0; rq < 9; rq++) {
 					const int dj = rq % 3 - 1, dk = rq / 3 - 1;
 					const T *xq = xr + dj * px + dk * pxy;
-					const V2 am = ld_stream<V2>(Ar + (3 * rq) * pa, ob);
-					const V2 a0 = ld_stream<V2>(Ar + (3 * rq + 1) * pa, ob);
-					const V2 ap = ld_stream<V2>(Ar + (3 * rq + 2) * pa, ob);
+					const V2 am = coef_or_zero<V2, X>(Ar, 3 * rq, pa, ob);
+					const V2 a0 = coef_or_zero<V2, X>(Ar, 3 * rq + 1, pa, ob);
+					const V2 ap = coef_or_zero<V2, X>(Ar, 3 * rq + 2, pa, ob);
 					const V2 xv = ld_row<V2>(xq, ob);
 					const T xm = ld_row<T>(xq - 1, ob);
 					const T xp = two ? ld_row<T>(xq + 2, ob) : (T)0;
@@ -1892,6 +1939,7 @@ __device__ __forceinline__ double residual_row_pair(const LevelView &L, const T 
 // FP32 residual with four points per lane (16-byte loads): segments of 256
 // points, the last one up to 257 with lane 63 doing the point out; the
 // wavefront does segment seg of row q.
+template <bool X>
 __device__ __forceinline__ double residual_row_quad_f32(const LevelView &L, const float *__restrict__ A,
 							const float *__restrict__ x, const float *__restrict__ r,
 							float *__restrict__ res, int q, int seg) {
@@ -1940,9 +1988,9 @@ __device__ __forceinline__ double residual_row_quad_f32(const LevelView &L, cons
 				for (int rq = 0; rq < 9; rq++) {
 					const int dj = rq % 3 - 1, dk = rq / 3 - 1;
 					const float *xq = xr + dj * px + dk * pxy;
-					const float4 am = ld_stream<float4>(Ar + (3 * rq) * pa, ob);
-					const float4 ac = ld_stream<float4>(Ar + (3 * rq + 1) * pa, ob);
-					const float4 ap = ld_stream<float4>(Ar + (3 * rq + 2) * pa, ob);
+					const float4 am = coef_or_zero<float4, X>(Ar, 3 * rq, pa, ob);
+					const float4 ac = coef_or_zero<float4, X>(Ar, 3 * rq + 1, pa, ob);
+					const float4 ap = coef_or_zero<float4, X>(Ar, 3 * rq + 2, pa, ob);
 					const float4 xv = ld_row<float4>(xq, ob);
 					const float xm = ld_row<float>(xq - 1, ob);
 					const float xp = nv == 4 ? ld_row<float>(xq + 4, ob) : 0.0f;
@@ -1984,23 +2032,18 @@ __device__ __forceinline__ double residual_row_quad_f32(const LevelView &L, cons
 
 // Residual rows, dispatched on the arithmetic type: four points per lane in
 // FP32 (residual into FP32), two in FP64.
-template <typename T, typename TR>
+template <typename T, typename TR, bool X>
 __device__ __forceinline__ double residual_row(const LevelView &L, const T *__restrict__ A, const T *__restrict__ x,
 					       const T *__restrict__ r, TR *__restrict__ res, int q, int seg,
 					       TR *__restrict__ zx = nullptr) {
-	return residual_row_pair<T, TR>(L, A, x, r, res, q, seg, zx);
-}
-template <>
-__device__ __forceinline__ double residual_row<float, float>(const LevelView &L, const float *__restrict__ A,
-							     const float *__restrict__ x, const float *__restrict__ r,
-							     float *__restrict__ res, int q, int seg, float *__restrict__ zx) {
-	return residual_row_quad_f32(L, A, x, r, res, q, seg);  // zx: not used in FP32
+	if constexpr (sizeof(T) == 4) return residual_row_quad_f32<X>(L, A, x, r, res, q, seg);  // zx: not used in FP32
+	else return residual_row_pair<T, TR, X>(L, A, x, r, res, q, seg, zx);
 }
 
 // Wavefront w of a residual launch: rows w*rpw .. when they fit the lanes,
 // else one segment of a long row (residual_segments per row).  w must be
 // wavefront-uniform.
-template <typename T, typename TR>
+template <typename T, typename TR, bool X = false>
 __device__ __forceinline__ double residual_wave(const LevelView &L, const T *__restrict__ A, const T *__restrict__ x,
 						const T *__restrict__ r, TR *__restrict__ res, TR *__restrict__ zx, int w) {
 	const int rows = L.n * L.o;
@@ -2008,21 +2051,21 @@ __device__ __forceinline__ double residual_wave(const LevelView &L, const T *__r
 	if (W.lpr <= 64) {
 		const int q0 = w * W.rpw;
 		if (q0 >= rows) return 0.0;
-		if constexpr (sizeof(T) == 8) return residual_lanes<T, TR, Ppl<T>::v, PO_ROWS>(L, A, x, r, res, zx, q0, rows);
+		if constexpr (sizeof(T) == 8) return residual_lanes<T, TR, Ppl<T>::v, PO_ROWS, X>(L, A, x, r, res, zx, q0, rows);
 		// FP32 point outs come with a tail copy (m = 4q+1)
-		if (W.ext) return residual_lanes<T, TR, Ppl<T>::v, PO_TAIL>(L, A, x, r, res, zx, q0, rows);
-		return residual_lanes<T, TR, Ppl<T>::v, PO_NONE>(L, A, x, r, res, zx, q0, rows);
+		if (W.ext) return residual_lanes<T, TR, Ppl<T>::v, PO_TAIL, X>(L, A, x, r, res, zx, q0, rows);
+		return residual_lanes<T, TR, Ppl<T>::v, PO_NONE, X>(L, A, x, r, res, zx, q0, rows);
 	}
 	const int nseg = residual_segments(L.m, (int)sizeof(T));
-	return residual_row<T, TR>(L, A, x, r, res, w / nseg, w % nseg, zx);
+	return residual_row<T, TR, X>(L, A, x, r, res, w / nseg, w % nseg, zx);
 }
 
-template <typename T, typename TR>
+template <typename T, typename TR, bool X>
 __global__ __launch_bounds__(256) void k_residual(LevelView L, const T *__restrict__ A, const T *__restrict__ x,
 						  const T *__restrict__ r, TR *__restrict__ res, double *__restrict__ partial,
 						  TR *__restrict__ zx) {
 	const int qb = xcd_block((int)blockIdx.x, (int)gridDim.x);
-	const double v2 = residual_wave<T, TR>(L, A, x, r, res, zx, __builtin_amdgcn_readfirstlane(qb * 4 + (int)threadIdx.y));
+	const double v2 = residual_wave<T, TR, X>(L, A, x, r, res, zx, __builtin_amdgcn_readfirstlane(qb * 4 + (int)threadIdx.y));
 	if (partial) {
 		// indexed by the block's logical number, so the sum order is that
 		// of a batched launch
@@ -2034,7 +2077,7 @@ __global__ __launch_bounds__(256) void k_residual(LevelView L, const T *__restri
 // Residual of a level with periodic axes, one point per thread, after the
 // halo holds the ghost copies: the 27-entry sum in box order from zero,
 // centre included (region.cc:1833-1842), as the row kernels form it.
-template <typename T, typename TR>
+template <typename T, typename TR, bool X>
 __global__ __launch_bounds__(256) void k_residual_pt(LevelView L, const T *__restrict__ A, const T *__restrict__ x,
 						     const T *__restrict__ r, TR *__restrict__ res,
 						     double *__restrict__ partial, TR *__restrict__ zx) {
@@ -2047,7 +2090,8 @@ __global__ __launch_bounds__(256) void k_residual_pt(LevelView L, const T *__res
 #pragma unroll
 		for (int e = 0; e < 27; e++) {
 			const int di = e % 3 - 1, dj = (e / 3) % 3 - 1, dk = e / 9 - 1;
-			ax = ax + Ap[e * L.pa] * x[p + di + dj * px + dk * pxy];
+			const T a = X && !in_cross(e) ? (T)0 : Ap[e * L.pa];
+			ax = ax + a * x[p + di + dj * px + dk * pxy];
 		}
 		const T v = r[p] - ax;
 		if (res) res[p] = (TR)v;
@@ -2074,12 +2118,14 @@ int launch_residual(hipStream_t s, const LevelView &L, const T *A, const T *x, c
 		// leaves its value unchanged
 		launch_halo_wrap<T>(s, L, const_cast<T *>(x));
 		dim3 grid((L.m + 63) / 64, (L.n + 3) / 4, L.o), block(64, 4, 1);
-		hipLaunchKernelGGL((k_residual_pt<T, TR>), grid, block, 0, s, L, A, x, r, res, partial, zero_out);
+		if (L.cross) hipLaunchKernelGGL((k_residual_pt<T, TR, true>), grid, block, 0, s, L, A, x, r, res, partial, zero_out);
+		else hipLaunchKernelGGL((k_residual_pt<T, TR, false>), grid, block, 0, s, L, A, x, r, res, partial, zero_out);
 		HIPCHECK_LAUNCH();
 		return residual_partial_count(L);
 	}
 	const int G = residual_blocks(L, (int)sizeof(T));
-	hipLaunchKernelGGL((k_residual<T, TR>), dim3(G), dim3(64, 4, 1), 0, s, L, A, x, r, res, partial, zero_out);
+	if (L.cross) hipLaunchKernelGGL((k_residual<T, TR, true>), dim3(G), dim3(64, 4, 1), 0, s, L, A, x, r, res, partial, zero_out);
+	else hipLaunchKernelGGL((k_residual<T, TR, false>), dim3(G), dim3(64, 4, 1), 0, s, L, A, x, r, res, partial, zero_out);
 	HIPCHECK_LAUNCH();
 	return G;
 }
@@ -2109,6 +2155,7 @@ int launch_sumsq(hipStream_t s, const LevelView &L, const T *r, double *partial)
 // array, region.cc:1861-1869, used by region::Ax): the 27-entry sum in box
 // order from zero.  in must have a zero halo on non-periodic axes and the
 // ghost copies on periodic ones.
+template <bool X>
 __global__ __launch_bounds__(256) void k_apply(LevelView L, const double *__restrict__ A, const double *__restrict__ in,
 					       double *__restrict__ out) {
 	const int i = (int)(blockIdx.x * 64 + threadIdx.x), j = (int)(blockIdx.y * 4 + threadIdx.y), k = (int)blockIdx.z;
@@ -2119,14 +2166,16 @@ __global__ __launch_bounds__(256) void k_apply(LevelView L, const double *__rest
 #pragma unroll
 	for (int e = 0; e < 27; e++) {
 		const int di = e % 3 - 1, dj = (e / 3) % 3 - 1, dk = e / 9 - 1;
-		ax = ax + Ap[e * L.pa] * in[p + di + dj * px + dk * pxy];
+		const double a = X && !in_cross(e) ? 0.0 : Ap[e * L.pa];
+		ax = ax + a * in[p + di + dj * px + dk * pxy];
 	}
 	out[p] = ax;
 }
 
 void launch_apply(hipStream_t s, const LevelView &L, const double *A, const double *in, double *out) {
 	dim3 grid((L.m + 63) / 64, (L.n + 3) / 4, L.o), block(64, 4, 1);
-	hipLaunchKernelGGL(k_apply, grid, block, 0, s, L, A, in, out);
+	if (L.cross) hipLaunchKernelGGL(k_apply<true>, grid, block, 0, s, L, A, in, out);
+	else hipLaunchKernelGGL(k_apply<false>, grid, block, 0, s, L, A, in, out);
 	HIPCHECK_LAUNCH();
 }
 
@@ -3290,12 +3339,18 @@ __global__ void k_unpack_vec(LevelView L, const double *__restrict__ d, double *
 	const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
 	if (t < n) c[t] = d[compact_to_padded(L, p0 + t)];
 }
-__global__ void k_pack_op(LevelView L, const double *__restrict__ c, double *__restrict__ A, long long p0, long long n) {
+__global__ void k_pack_op(LevelView L, const double *__restrict__ c, double *__restrict__ A, long long p0, long long n,
+			  int *dense) {
 	const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
 	if (t >= n * 27) return;
 	const int e = (int)(t % 27);
 	const long long p = t / 27;
-	A[compact_to_coef(L, e, p0 + p)] = c[t];
+	const double v = c[t];
+	A[compact_to_coef(L, e, p0 + p)] = v;
+	// every writer stores the same 1; the test spares a dense operator one
+	// store per entry to a single line (a NaN entry counts as nonzero)
+	if (dense && !in_cross(e) && !(v == 0.0) && __hip_atomic_load(dense, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+		__hip_atomic_store(dense, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __global__ void k_unpack_op(LevelView L, const double *__restrict__ A, double *__restrict__ c, long long p0, long long n) {
 	const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -3315,8 +3370,8 @@ void launch_unpack_vec(hipStream_t s, const LevelView &L, const double *d, doubl
 	if (n > 0) hipLaunchKernelGGL(k_unpack_vec, dim3(nblk(n, 256)), dim3(256), 0, s, L, d, c, p0, n);
 	HIPCHECK_LAUNCH();
 }
-void launch_pack_op(hipStream_t s, const LevelView &L, const double *c, double *A, long long p0, long long n) {
-	if (n > 0) hipLaunchKernelGGL(k_pack_op, dim3(nblk(n * 27, 256)), dim3(256), 0, s, L, c, A, p0, n);
+void launch_pack_op(hipStream_t s, const LevelView &L, const double *c, double *A, long long p0, long long n, int *dense) {
+	if (n > 0) hipLaunchKernelGGL(k_pack_op, dim3(nblk(n * 27, 256)), dim3(256), 0, s, L, c, A, p0, n, dense);
 	HIPCHECK_LAUNCH();
 	launch_coef_tail(s, L, A);
 }
