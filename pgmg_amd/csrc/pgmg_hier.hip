@@ -251,10 +251,43 @@ void skew_sweeps(pgmg_hier *h, Level &L, int nsweeps) {
 		launch_gs_planes_skew<T>(h->stream, L.sv, sA<T>(L), sx<T>(L), sr<T>(L), nsweeps);
 }
 
-// from_zero: x is 0 on entry (and may not be cleared in memory); only with
-// gs_from_zero_ok.
+// Whether a level's forward colour sweeps run as one launch each
+// (launch_gs_tile), back and forth between x and the residual scratch.
 template <typename T>
-void op_gs(pgmg_hier *h, int level, int mode, int nsweeps, bool from_zero = false) {
+bool gs_use_tile(const pgmg_hier *h, int level, int mode) {
+	const Level &L = h->lev[level];
+	return h->opts.smoother != PGMG_SMOOTH_EXACT && !mode && !gs_use_small<T>(h, L, mode) && gs_tile_ok<T>(L.v);
+}
+
+// Where x is when a smoothing call starts: in the level's x, in the residual
+// scratch, or known to be 0 (and possibly not cleared in memory).  X_SCRATCH
+// only with gs_use_tile, X_ZERO with gs_from_zero_ok or gs_use_tile.
+enum XStart { X_LEVEL, X_SCRATCH, X_ZERO };
+
+template <typename T>
+void tile_sweeps(pgmg_hier *h, int level, int nsweeps, XStart from) {
+	Level &L = h->lev[level];
+	T *x = lx<T>(L), *other = res_scratch<T>(h);
+	int left = nsweeps;
+	if (from == X_LEVEL && (left & 1)) {
+		// an odd number of exchanges would leave x in the scratch: one
+		// sweep in place
+		ProfScope ps(h, KC_GS, level, L.points());
+		for (int q = 0; q < 4; q++) launch_gs_pair<T>(h->stream, L.v, lA<T>(L), x, lr<T>(L), q, false);
+		left--;
+	}
+	const T *in = from == X_ZERO ? nullptr : from == X_SCRATCH ? other : x;
+	for (; left > 0; left--) {
+		T *out = (left & 1) ? x : other;  // the last sweep writes x
+		ProfScope ps(h, KC_GS, level, L.points());
+		launch_gs_tile<T>(h->stream, L.v, lA<T>(L), in, out, lr<T>(L));
+		in = out;
+	}
+}
+
+template <typename T>
+void op_gs(pgmg_hier *h, int level, int mode, int nsweeps, XStart from = X_LEVEL) {
+	const bool from_zero = from == X_ZERO;
 	Level &L = h->lev[level];
 	const bool exact = h->opts.smoother == PGMG_SMOOTH_EXACT;
 	h->gs_count += nsweeps;
@@ -303,6 +336,10 @@ void op_gs(pgmg_hier *h, int level, int mode, int nsweeps, bool from_zero = fals
 	if (use_small) {
 		ProfScope ps(h, KC_GS, level, L.points() * nsweeps * (mode ? 2 : 1));
 		launch_gs_small<T>(h->stream, L.v, lA<T>(L), lx<T>(L), lr<T>(L), nsweeps, mode, exact ? 1 : 0);
+		return;
+	}
+	if (gs_use_tile<T>(h, level, mode)) {
+		tile_sweeps<T>(h, level, nsweeps, from);
 		return;
 	}
 	const int tmax = (L.v.m - 1) + 2 * (L.v.n - 1) + 4 * (L.v.o - 1);
@@ -367,10 +404,10 @@ void op_restriction(pgmg_hier *h, int level) {
 }
 
 template <typename T>
-void op_interpolation(pgmg_hier *h, int level) {
+void op_interpolation(pgmg_hier *h, int level, bool to_scratch = false) {
 	Level &C = h->lev[level], &F = h->lev[level - 1];
 	ProfScope ps(h, KC_INTERP, level, F.points());
-	launch_interp<T>(h->stream, C.v, F.v, lx<T>(C), lx<T>(F));
+	launch_interp<T>(h->stream, C.v, F.v, lx<T>(C), lx<T>(F), to_scratch ? res_scratch<T>(h) : lx<T>(F));
 }
 
 template <typename T>
@@ -389,13 +426,19 @@ template <typename T>
 void op_v_cycle(pgmg_hier *h, int mode, bool top_zero = false) {
 	const int L = h->nl;
 	for (int i = 0; i < L - 1; i++) {
-		op_gs<T>(h, i, mode, h->opts.v_down + i, top_zero && i == 0);
+		// below level 0 the restriction cleared x
+		const bool zero = i == 0 ? top_zero : gs_use_tile<T>(h, i, mode);
+		op_gs<T>(h, i, mode, h->opts.v_down + i, zero ? X_ZERO : X_LEVEL);
 		op_restriction<T>(h, i + 1);
 	}
 	op_solve_exact<T>(h, L - 1, false);
 	for (int i = L - 1; i > 0; i--) {
-		op_interpolation<T>(h, i);
-		op_gs<T>(h, i - 1, mode, h->opts.v_up + i - 1);
+		// an odd number of launch_gs_tile sweeps starts from the scratch, to
+		// end in x
+		const int sweeps = h->opts.v_up + i - 1;
+		const bool odd = (sweeps & 1) && gs_use_tile<T>(h, i - 1, mode);
+		op_interpolation<T>(h, i, odd);
+		op_gs<T>(h, i - 1, mode, sweeps, odd ? X_SCRATCH : X_LEVEL);
 	}
 }
 

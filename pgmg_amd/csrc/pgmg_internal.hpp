@@ -270,6 +270,11 @@ template <typename T> void launch_gs_colour(hipStream_t s, const LevelView &L, c
 // x need not be cleared beforehand.
 template <typename T> void launch_gs_pair(hipStream_t s, const LevelView &L, const T *A, T *x, const T *r, int pair,
 					  bool from_zero = false);
+// One forward eight-colour sweep of a small level (gs_tile_ok) in one launch:
+// xout = the sweep of xin, which may be null for an x of zeros.  xin and xout
+// are different arrays in L's layout; only grid points of them are accessed.
+template <typename T> bool gs_tile_ok(const LevelView &L);
+template <typename T> void launch_gs_tile(hipStream_t s, const LevelView &L, const T *A, const T *xin, T *xout, const T *r);
 // Ghost copies of the wrapped points into the halo of the periodic axes of
 // L (no-op without periodic axes).
 template <typename T> void launch_halo_wrap(hipStream_t s, const LevelView &L, T *x);
@@ -325,8 +330,9 @@ void launch_reduce(hipStream_t s, const double *partial, int n, double *out);
 template <typename T> int launch_sumsq(hipStream_t s, const LevelView &L, const T *r, double *partial);
 // rc = R res (gather form of the reference's scatter), xc = 0.
 template <typename T> void launch_restrict(hipStream_t s, const LevelView &F, const LevelView &C, const T *res, T *rc, T *xc);
-// xf += P xc.
-template <typename T> void launch_interp(hipStream_t s, const LevelView &C, const LevelView &F, const T *xc, T *xf);
+// xo = xf + P xc at the grid points of F (xo may be xf).
+template <typename T> void launch_interp(hipStream_t s, const LevelView &C, const LevelView &F, const T *xc, const T *xf,
+					 T *xo);
 // Ac = P^T Af P / 8.
 void launch_rat(hipStream_t s, const LevelView &F, const LevelView &C, const double *Af, double *Ac);
 // Dense bottom LU.

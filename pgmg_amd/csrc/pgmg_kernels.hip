@@ -1013,6 +1013,219 @@ void launch_gs_pair(hipStream_t s, const LevelView &L, const T *A, T *x, const T
 	HIPCHECK_LAUNCH();
 }
 
+// One forward eight-colour sweep of a small level in one launch.  Such a
+// level is bound by latency, not by bytes: k_gs_pair takes four launches a
+// sweep at about 3.6 us each whatever the level's size.
+//
+// A workgroup owns a tile of kTileJ rows (j) x kTileK planes (k) of whole rows
+// in i.  It stages x of the tile and the rows around it in LDS and runs the
+// colour pairs p = (cj,ck), in the order (0,0), (1,0), (0,1), (1,1), between
+// barriers.  The rows outside the tile whose new values its own rows read it
+// updates itself, from the same inputs in the same order, so every tile has
+// the bits of a sweep over the whole level.  Other tiles read the old x of its
+// rows, so the new x goes to another array.  Pair p covers rows j = J0-2+p ..
+// J1+2-p and planes k = K0+ck .. K1-ck of the tile [J0,J1) x [K0,K1) (step 2
+// each), from the old x of j = J0-3 .. J1+3, k = K0-1 .. K1+1: 23 rows for the
+// 8 of a 4 x 2 tile.  More rows a tile (8 x 2: 35 rows for 16) lose more to the
+// 64 bytes a clock of their CU's loads than the fewer repeated rows save.
+//
+// Every wavefront belongs to one colour pair, and each of its threads holds
+// one point pair (i0, i0+1), i0 even, of one row, with its 27 coefficients in
+// registers from the start: all loads of the launch go out at once, one round
+// trip.  Even points update first, together with the odd points' terms that
+// no new even value enters, the odd ones after a barrier.  Per-point
+// arithmetic and order as in gs_point.  Indices are 32-bit with 24-bit
+// products, and the host passes what it can work out (TileGeom).
+// Only grid points of xin and xout are accessed (their halos may hold
+// anything), and positions outside the grid count as 0 (loaded from r's
+// first, halo, element), so the level must not be periodic.
+//
+// Measured, launches back to back: 17^3 6.5 us a sweep against 14.5 (FP32;
+// FP64 6.7 against 14.9), 33^3 6.8 against 14.5 (FP64 7.2 against 14.7); 65^3,
+// whose 561 tiles are more than two to a CU, 24 against 16 (not used there).
+constexpr int kTileJ = 4, kTileK = 2;
+struct TileGeom {
+	int m, n, o, px, pxy, base;  // as LevelView, 32-bit
+	int pa, ablk;                // coefficient row and block pitch
+	int tj, tiles;               // tiles along j, and in all
+	int hx, nh;                  // x in LDS: row length, elements
+	int si, sj, sk;              // the thread count in LDS rows and planes: nt = si + hx*(sj + kTileHy*sk)
+	int np;                      // point pairs a row
+	int w1, w2, w3, w4;          // first wavefront of pairs 1, 2, 3; wavefronts in all
+	float inv_np, inv_hx;
+};
+constexpr int kTileHy = kTileJ + 7, kTileHz = kTileK + 3;  // rows and planes of x in LDS
+// Rows and planes of colour pair p in a tile.
+__host__ __device__ constexpr int tile_nj(int p) { return kTileJ / 2 + 3 - p; }
+__host__ __device__ constexpr int tile_nk(int p) { return kTileK / 2 + 1 - (p >> 1); }
+
+// a / b for 0 <= a < 2^20, from inv = 1/b rounded: (a + 0.5) / b is at least
+// 0.5/b away from a whole number, more than the rounding errors.
+__device__ __forceinline__ int div_small(int a, float inv) { return (int)(((float)a + 0.5f) * inv); }
+
+constexpr int kTileStage = 6;
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void k_gs_tile(TileGeom G, const T *__restrict__ A, const T *__restrict__ xin,
+						T *__restrict__ xout, const T *__restrict__ r) {
+	typedef typename Vec2<T>::type V2;
+	extern __shared__ __align__(16) char smem_[];
+	T *xs = (T *)smem_;
+	const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
+	const int tk = tile / G.tj;
+	const int J0 = (tile - tk * G.tj) * kTileJ, K0 = tk * kTileK;
+	const int hxy = G.hx * kTileHy;
+	const int jb = J0 - 3, kb = K0 - 1;  // first row and plane staged
+	const int tid = threadIdx.x;
+	// x into LDS: the loads first, so that writing them does not wait for
+	// the coefficients (xin null: x is 0)
+	const int row0 = div_small(tid, G.inv_hx);
+	int si = tid - __mul24(row0, G.hx), sk = row0 / kTileHy, sj = row0 - sk * kTileHy;
+	auto stage = [&]() -> T {
+		// LDS position (si, sj, sk) is grid point (si-1, jb+sj, kb+sk)
+		const int j = jb + sj, k = kb + sk;
+		const bool in = xin && (unsigned)(si - 1) < (unsigned)G.m && (unsigned)j < (unsigned)G.n && (unsigned)k < (unsigned)G.o;
+		const int off = in ? G.base + si - 1 + __mul24(j, G.px) + __mul24(k, G.pxy) : 0;
+		const T v = (in ? xin : r)[off];
+		si += G.si; sj += G.sj; sk += G.sk;
+		if (si >= G.hx) { si -= G.hx; sj++; }
+		if (sj >= kTileHy) { sj -= kTileHy; sk++; }
+		return v;
+	};
+	T xv[kTileStage];
+#pragma unroll
+	for (int u = 0; u < kTileStage; u++) xv[u] = stage();
+	// this thread's colour pair and point pair
+	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const int my = wave >= G.w4 ? -1 : wave >= G.w3 ? 3 : wave >= G.w2 ? 2 : wave >= G.w1 ? 1 : 0;
+	const int w0 = my == 3 ? G.w3 : my == 2 ? G.w2 : my == 1 ? G.w1 : 0;
+	bool live = false, two = false, own = false;
+	int lq = hxy + 1;  // the even point's place in LDS
+	uint32_t xo = 0;
+	V2 c[27], rv;
+	if (my >= 0) {
+		const int ck = my >> 1, nj = tile_nj(my);
+		const int it = tid - 64 * w0;
+		const int row = div_small(it, G.inv_np), i0 = 2 * (it - __mul24(row, G.np));
+		const int kr = div_small(row, 1.0f / (float)nj), jr = row - __mul24(kr, nj);
+		const int j = J0 - 2 + my + 2 * jr, k = K0 + ck + 2 * kr;
+		if (kr < tile_nk(my) && (unsigned)j < (unsigned)G.n && (unsigned)k < (unsigned)G.o) {
+			live = true;
+			two = i0 + 1 < G.m;
+			own = j >= J0 && j < J0 + kTileJ && k < K0 + kTileK;
+			lq = (i0 + 1) + __mul24(G.hx, j - jb) + __mul24(hxy, k - kb);
+			xo = (uint32_t)(G.base + i0 + __mul24(j, G.px) + __mul24(k, G.pxy)) * (uint32_t)sizeof(T);
+			const uint32_t ao = (uint32_t)(i0 + __mul24(G.ablk, j + 1 + __mul24(G.n + 2, k + 1))) * (uint32_t)sizeof(T);
+			rv = ld_row<V2>(r, xo);
+#pragma unroll
+			for (int e = 0; e < 27; e++) c[e] = ld_row<V2>(A + e * G.pa, ao);
+		}
+	}
+#pragma unroll
+	for (int u = 0; u < kTileStage; u++)
+		if (tid + u * NT < G.nh) xs[tid + u * NT] = xv[u];
+	for (int q = tid + kTileStage * NT; q < G.nh; q += NT) xs[q] = stage();
+	__syncthreads();
+	T *xl = xs + lq;
+	T xe = (T)0, xd = (T)0;
+	for (int p = 0; p < 4; p++) {
+		const bool on = my == p && live;
+		T ay = (T)0, iy = (T)0;
+		T prod[12];
+		if (on) {
+			T ax = (T)0;
+#pragma unroll
+			for (int rq = 0; rq < 9; rq++) {
+				const T *xr = xl + (rq % 3 - 1) * G.hx + (rq / 3 - 1) * hxy;
+				const V2 xa = *(const V2 *)(xr - 1), xb = *(const V2 *)(xr + 1);
+				const V2 am = c[3 * rq], a0 = c[3 * rq + 1], ap = c[3 * rq + 2];
+				ax = ax + am.x * xa.x;
+				if (rq != 4) ax = ax + a0.x * xa.y;
+				ax = ax + ap.x * xb.x;
+				if (rq < 4) {
+					ay = ay + am.y * xa.y;
+					ay = ay + a0.y * xb.x;
+					ay = ay + ap.y * xb.y;
+				} else if (rq > 4) {
+					prod[3 * (rq - 5)] = am.y * xa.y;
+					prod[3 * (rq - 5) + 1] = a0.y * xb.x;
+					prod[3 * (rq - 5) + 2] = ap.y * xb.y;
+				}
+			}
+			xe = (rv.x - ax) * ((T)1 / c[13].x);
+			xl[0] = xe;
+			iy = (T)1 / c[13].y;
+		}
+		__syncthreads();
+		if (on && two) {
+			ay = ay + c[12].y * xe;
+			ay = ay + c[14].y * xl[2];
+#pragma unroll
+			for (int q = 0; q < 12; q++) ay = ay + prod[q];
+			xd = (rv.y - ay) * iy;
+			xl[1] = xd;
+		}
+		__syncthreads();
+	}
+	// the tile's own rows: each of its point pairs belongs to one thread
+	if (own) {
+		T *xp = (T *)((char *)xout + xo);
+		if (two) {
+			V2 v;
+			v.x = xe;
+			v.y = xd;
+			*(V2 *)xp = v;
+		} else {
+			*xp = xe;
+		}
+	}
+}
+
+// The launch of k_gs_tile on level L; false where the level does not take it:
+// periodic, more tiles than CUs (two or more to a CU run one after the other),
+// or rows too long for a tile to have a thread a point pair (16 wavefronts
+// of 128 registers in FP32, 12 of 168 in FP64) or for its x to fit LDS.
+template <typename T>
+bool tile_geom(const LevelView &L, TileGeom &G, int &nt, size_t &lds) {
+	if (L.prd) return false;
+	G.np = (L.m + 1) / 2;
+	int w[5] = {0, 0, 0, 0, 0};
+	for (int p = 0; p < 4; p++) w[p + 1] = w[p] + (tile_nj(p) * tile_nk(p) * G.np + 63) / 64;
+	G.hx = (L.m + 3) & ~1;  // i = -1 .. m+1, even: the pairs (i0-1, i0) and (i0+1, i0+2) are aligned
+	G.tj = (L.n + kTileJ - 1) / kTileJ;
+	const long long tiles = (long long)G.tj * ((L.o + kTileK - 1) / kTileK), nh = (long long)G.hx * kTileHy * kTileHz;
+	if (w[4] > (sizeof(T) == 4 ? 16 : 12) || nh * (long long)sizeof(T) > kSmallLdsBytes || tiles > 256) return false;
+	nt = w[4] <= 8 ? 512 : sizeof(T) == 4 ? 1024 : 768;
+	lds = sizeof(T) * (size_t)nh;
+	G.tiles = (int)tiles;
+	G.nh = (int)nh;
+	G.w1 = w[1]; G.w2 = w[2]; G.w3 = w[3]; G.w4 = w[4];
+	G.m = L.m; G.n = L.n; G.o = L.o; G.px = L.px; G.pxy = (int)L.pxy; G.base = (int)L.base;
+	G.pa = L.pa; G.ablk = (int)ablock(L);
+	G.si = nt % G.hx; G.sj = nt / G.hx % kTileHy; G.sk = nt / G.hx / kTileHy;
+	G.inv_np = 1.0f / (float)G.np; G.inv_hx = 1.0f / (float)G.hx;
+	return true;
+}
+
+template <typename T>
+bool gs_tile_ok(const LevelView &L) {
+	TileGeom G;
+	int nt;
+	size_t lds;
+	return tile_geom<T>(L, G, nt, lds);
+}
+
+template <typename T>
+void launch_gs_tile(hipStream_t s, const LevelView &L, const T *A, const T *xin, T *xout, const T *r) {
+	TileGeom G;
+	int nt = 0;
+	size_t lds = 0;
+	if (!tile_geom<T>(L, G, nt, lds)) return;
+	constexpr int kMost = sizeof(T) == 4 ? 1024 : 768;
+	if (nt == 512) hipLaunchKernelGGL((k_gs_tile<T, 512>), dim3(G.tiles), dim3(512), lds, s, G, A, xin, xout, r);
+	else hipLaunchKernelGGL((k_gs_tile<T, kMost>), dim3(G.tiles), dim3(kMost), lds, s, G, A, xin, xout, r);
+	HIPCHECK_LAUNCH();
+}
+
 // Hyperplane i + 2j + 4k = t.  Every stencil offset (di,dj,dk) != 0 has
 // di + 2dj + 4dk != 0, negative exactly for the offsets that precede the
 // centre in lexicographic order; sweeping t upwards therefore gives each
@@ -2553,7 +2766,7 @@ __device__ __forceinline__ T interp_value(int pos, bool full, bool xs, bool ys, 
 // (up to) eight fine points updated as four x pairs (2ic, 2ic+1).
 template <typename T>
 __device__ __forceinline__ void interp_cube(const LevelView &C, const LevelView &F, const T *__restrict__ xc,
-					    T *__restrict__ xf, int ic, int jc, int kc) {
+					    const T *xf, T *xo, int ic, int jc, int kc) {
 	typedef typename Vec2<T>::type V2;
 	const int lastx = (F.m - 1) >> 1, lasty = (F.n - 1) >> 1, lastz = (F.o - 1) >> 1;
 	// on a periodic axis the upper neighbour of the last cube is coarse 0
@@ -2585,26 +2798,26 @@ __device__ __forceinline__ void interp_cube(const LevelView &C, const LevelView 
 				V2 f = *(const V2 *)(xf + p);
 				f.x = f.x + a;
 				f.y = f.y + b;
-				*(V2 *)(xf + p) = f;
+				*(V2 *)(xo + p) = f;
 			} else {
-				xf[p] = xf[p] + a;
+				xo[p] = xf[p] + a;
 			}
 		}
 	}
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_interp(LevelView C, LevelView F, const T *__restrict__ xc, T *__restrict__ xf) {
+__global__ __launch_bounds__(256) void k_interp(LevelView C, LevelView F, const T *__restrict__ xc, const T *xf, T *xo) {
 	const int ic = (int)(blockIdx.x * 64 + threadIdx.x), jc = (int)(blockIdx.y * 4 + threadIdx.y), kc = (int)blockIdx.z;
 	if (ic >= (F.m + 1) / 2 || jc >= (F.n + 1) / 2) return;
-	interp_cube<T>(C, F, xc, xf, ic, jc, kc);
+	interp_cube<T>(C, F, xc, xf, xo, ic, jc, kc);
 }
 
 template <typename T>
-void launch_interp(hipStream_t s, const LevelView &C, const LevelView &F, const T *xc, T *xf) {
+void launch_interp(hipStream_t s, const LevelView &C, const LevelView &F, const T *xc, const T *xf, T *xo) {
 	const int ncx = (F.m + 1) / 2, ncy = (F.n + 1) / 2, ncz = (F.o + 1) / 2;
 	dim3 grid((ncx + 63) / 64, (ncy + 3) / 4, ncz), block(64, 4, 1);
-	hipLaunchKernelGGL(k_interp<T>, grid, block, 0, s, C, F, xc, xf);
+	hipLaunchKernelGGL(k_interp<T>, grid, block, 0, s, C, F, xc, xf, xo);
 	HIPCHECK_LAUNCH();
 }
 
@@ -3600,7 +3813,7 @@ __global__ __launch_bounds__(256) void kb_interp(const SlotDev *__restrict__ slo
 	BATCH_LOOP
 		const LevelView F = S->lv[level - 1];
 		int ic, jc, kc;
-		if (cubes_unit(F, lu, ic, jc, kc)) interp_cube<T>(S->lv[level], F, sx<T>(S, level), sx<T>(S, level - 1), ic, jc, kc);
+		if (cubes_unit(F, lu, ic, jc, kc)) interp_cube<T>(S->lv[level], F, sx<T>(S, level), sx<T>(S, level - 1), sx<T>(S, level - 1), ic, jc, kc);
 	}
 }
 
@@ -3708,7 +3921,9 @@ void launch_b_add_x(hipStream_t s, const SlotDev *slots, WorkList wl, int chunk)
 	template void launch_gs_small<T>(hipStream_t, const LevelView &, const T *, T *, const T *, int, int, int); \
 	template int launch_sumsq<T>(hipStream_t, const LevelView &, const T *, double *); \
 	template void launch_restrict<T>(hipStream_t, const LevelView &, const LevelView &, const T *, T *, T *); \
-	template void launch_interp<T>(hipStream_t, const LevelView &, const LevelView &, const T *, T *); \
+	template void launch_interp<T>(hipStream_t, const LevelView &, const LevelView &, const T *, const T *, T *); \
+	template void launch_gs_tile<T>(hipStream_t, const LevelView &, const T *, const T *, T *, const T *); \
+	template bool gs_tile_ok<T>(const LevelView &); \
 	template void launch_lu_solve<T>(hipStream_t, const LevelView &, int, const double *, const int *, const T *, T *); \
 	template void launch_fill<T>(hipStream_t, T *, long long, T); \
 	template void launch_b_gs_pair<T>(hipStream_t, const SlotDev *, WorkList, int, int, bool, int); \
