@@ -1044,6 +1044,71 @@ void launch_gs_pair(hipStream_t s, const LevelView &L, const T *A, T *x, const T
 // FP64 6.7 against 14.9), 33^3 6.8 against 14.5 (FP64 7.2 against 14.7); 65^3,
 // whose 561 tiles are more than two to a CU, 24 against 16 (not used there).
 constexpr int kTileJ = 4, kTileK = 2;
+// One colour pair of a level (or tile) with x in LDS: the threads that are on
+// update their point pair (i0, i0+1), xl its even point in LDS, from the pair's
+// coefficients c, r and reciprocal diagonals (ix, iy): the even point, and the
+// odd point's terms that no new even value enters, then after a barrier the odd
+// point (where the row has it: two).  Every thread must call it; barrier after
+// both.  The row pitch hx is even and xl - 1 aligned, so that the x of a row is
+// two vector reads.  Arithmetic and order as in gs_point.
+template <typename T, int NT>
+__device__ __forceinline__ void lds_pair_step(const typename Vec2<T>::type (&c)[27], typename Vec2<T>::type rv, T ix, T iy,
+					      T *xl, int hx, int hxy, bool on, bool two, T &xe, T &xd) {
+	typedef typename Vec2<T>::type V2;
+	T ay = (T)0;
+	T prod[12];
+	if (on) {
+		// the LDS reads of a group of rows go out together (left alone, the
+		// compiler reads a row, waits and sums, to save registers: 24 sweeps
+		// of 9^3 FP64 62 us, so 55); in FP64 as many as the registers of NT
+		// threads take without scratch
+		constexpr int kGroup = sizeof(T) == 4 ? 9 : NT <= 512 ? 5 : 3;
+		T ax = (T)0;
+#pragma unroll
+		for (int g = 0; g < 9; g += kGroup) {
+			V2 xa[kGroup], xb[kGroup];
+#pragma unroll
+			for (int q = 0; q < kGroup; q++) {
+				if (g + q > 8) break;
+				const T *xr = xl + ((g + q) % 3 - 1) * hx + ((g + q) / 3 - 1) * hxy;
+				xa[q] = *(const V2 *)(xr - 1);
+				xb[q] = *(const V2 *)(xr + 1);
+			}
+			__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+			for (int q = 0; q < kGroup; q++) {
+				const int rq = g + q;
+				if (rq > 8) break;
+				const V2 am = c[3 * rq], a0 = c[3 * rq + 1], ap = c[3 * rq + 2];
+				ax = ax + am.x * xa[q].x;
+				if (rq != 4) ax = ax + a0.x * xa[q].y;
+				ax = ax + ap.x * xb[q].x;
+				if (rq < 4) {
+					ay = ay + am.y * xa[q].y;
+					ay = ay + a0.y * xb[q].x;
+					ay = ay + ap.y * xb[q].y;
+				} else if (rq > 4) {
+					prod[3 * (rq - 5)] = am.y * xa[q].y;
+					prod[3 * (rq - 5) + 1] = a0.y * xb[q].x;
+					prod[3 * (rq - 5) + 2] = ap.y * xb[q].y;
+				}
+			}
+		}
+		xe = (rv.x - ax) * ix;
+		xl[0] = xe;
+	}
+	__syncthreads();
+	if (on && two) {
+		ay = ay + c[12].y * xe;
+		ay = ay + c[14].y * xl[2];
+#pragma unroll
+		for (int q = 0; q < 12; q++) ay = ay + prod[q];
+		xd = (rv.y - ay) * iy;
+		xl[1] = xd;
+	}
+	__syncthreads();
+}
+
 struct TileGeom {
 	int m, n, o, px, pxy, base;  // as LevelView, 32-bit
 	int pa, ablk;                // coefficient row and block pitch
@@ -1124,48 +1189,15 @@ __global__ __launch_bounds__(NT) void k_gs_tile(TileGeom G, const T *__restrict_
 	for (int u = 0; u < kTileStage; u++)
 		if (tid + u * NT < G.nh) xs[tid + u * NT] = xv[u];
 	for (int q = tid + kTileStage * NT; q < G.nh; q += NT) xs[q] = stage();
-	__syncthreads();
-	T *xl = xs + lq;
-	T xe = (T)0, xd = (T)0;
-	for (int p = 0; p < 4; p++) {
-		const bool on = my == p && live;
-		T ay = (T)0, iy = (T)0;
-		T prod[12];
-		if (on) {
-			T ax = (T)0;
-#pragma unroll
-			for (int rq = 0; rq < 9; rq++) {
-				const T *xr = xl + (rq % 3 - 1) * G.hx + (rq / 3 - 1) * hxy;
-				const V2 xa = *(const V2 *)(xr - 1), xb = *(const V2 *)(xr + 1);
-				const V2 am = c[3 * rq], a0 = c[3 * rq + 1], ap = c[3 * rq + 2];
-				ax = ax + am.x * xa.x;
-				if (rq != 4) ax = ax + a0.x * xa.y;
-				ax = ax + ap.x * xb.x;
-				if (rq < 4) {
-					ay = ay + am.y * xa.y;
-					ay = ay + a0.y * xb.x;
-					ay = ay + ap.y * xb.y;
-				} else if (rq > 4) {
-					prod[3 * (rq - 5)] = am.y * xa.y;
-					prod[3 * (rq - 5) + 1] = a0.y * xb.x;
-					prod[3 * (rq - 5) + 2] = ap.y * xb.y;
-				}
-			}
-			xe = (rv.x - ax) * ((T)1 / c[13].x);
-			xl[0] = xe;
-			iy = (T)1 / c[13].y;
-		}
-		__syncthreads();
-		if (on && two) {
-			ay = ay + c[12].y * xe;
-			ay = ay + c[14].y * xl[2];
-#pragma unroll
-			for (int q = 0; q < 12; q++) ay = ay + prod[q];
-			xd = (rv.y - ay) * iy;
-			xl[1] = xd;
-		}
-		__syncthreads();
+	T ix = (T)0, iy = (T)0;
+	if (live) {
+		ix = (T)1 / c[13].x;
+		iy = (T)1 / c[13].y;
 	}
+	__syncthreads();
+	T xe = (T)0, xd = (T)0;
+	for (int p = 0; p < 4; p++)
+		lds_pair_step<T, NT>(c, rv, ix, iy, xs + lq, G.hx, hxy, my == p && live, two, xe, xd);
 	// the tile's own rows: each of its point pairs belongs to one thread
 	if (own) {
 		T *xp = (T *)((char *)xout + xo);
@@ -2008,6 +2040,89 @@ __device__ __forceinline__ void gs_lds_body(const LevelView &L, const T *__restr
 		gs_lds_run<T, false>(L, A, x, r, nsweeps, mode, exact, xs);
 }
 
+// Forward colour sweeps of a level whose point pairs each get a thread of one
+// workgroup of NT threads, the pairs of a colour pair (0,cj,ck), (1,cj,ck) in
+// wavefronts of their own: x in LDS, coefficients in registers, two barriers
+// a colour pair (lds_pair_step).  The bottom level's 24 sweeps are a chain of
+// 96 such steps, so what counts is a step's length: 24 sweeps of 9^3 FP32
+// 65 -> 51 us, FP64 77 -> 55 us, against one class a barrier with a point a
+// thread and the diagonal divided by each time (gs_lds_run).
+// x's row pitch in LDS: i = -1 .. m+1, even.
+__host__ __device__ inline int pair_pitch(int m) { return (m + 3) & ~1; }
+__host__ __device__ inline long long pair_lds_bytes(const LevelView &L, int elem) {
+	return (long long)pair_pitch(L.m) * (L.n + 2) * (L.o + 2) * elem;
+}
+// Wavefronts of colour pair p.
+__host__ __device__ inline int pair_waves(const LevelView &L, int p) {
+	return (((L.m + 1) >> 1) * ((L.n - (p & 1) + 1) >> 1) * ((L.o - (p >> 1) + 1) >> 1) + 63) >> 6;
+}
+// Threads of the workgroup that takes level L, or 0.
+__host__ __device__ inline int pair_threads(const LevelView &L, int elem) {
+	if ((long long)L.m * L.n * L.o > 1024 || pair_lds_bytes(L, elem) > kSmallLdsBytes) return 0;
+	const int w = pair_waves(L, 0) + pair_waves(L, 1) + pair_waves(L, 2) + pair_waves(L, 3);
+	return w <= 8 ? 512 : w <= 12 ? 768 : 0;
+}
+
+template <typename T, int NT>
+__device__ __forceinline__ void gs_lds_pairs(const LevelView &L, const T *__restrict__ A, T *__restrict__ x,
+					     const T *__restrict__ r, int nsweeps, T *__restrict__ xs) {
+	typedef typename Vec2<T>::type V2;
+	const int tid = threadIdx.x;
+	const int hx = pair_pitch(L.m), hxy = hx * (L.n + 2), nh = hxy * (L.o + 2);
+	for (int q = tid; q < nh; q += NT) {
+		const int i = q % hx - 1, j = (q / hx) % (L.n + 2) - 1, k = q / hxy - 1;
+		xs[q] = x[idx3(L, i, j, k)];
+	}
+	const int np = (L.m + 1) >> 1;
+	int my = -1, lq = hxy + hx + 1;
+	bool live = false, two = false;
+	long long at = 0;
+	V2 c[27], rv;
+	T ix = (T)0, iy = (T)0;
+	int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+	for (int p = 0; p < 4; p++) {
+		const int pw = pair_waves(L, p);
+		if (my < 0 && w < pw) {
+			my = p;
+			const int cj = p & 1, ck = p >> 1, nb = (L.n - cj + 1) >> 1, nd = (L.o - ck + 1) >> 1;
+			const int it = 64 * w + (tid & 63), a = it % np, b = (it / np) % nb, d = it / (np * nb);
+			if (d < nd) {
+				const int i0 = 2 * a, j = 2 * b + cj, k = 2 * d + ck;
+				live = true;
+				two = i0 + 1 < L.m;
+				lq = (i0 + 1) + hx * (j + 1) + hxy * (k + 1);
+				at = idx3(L, i0, j, k);
+				rv = *(const V2 *)(r + at);
+				const T *Ap = A + aidx3(L, 0, i0, j, k);
+#pragma unroll
+				for (int e = 0; e < 27; e++) c[e] = *(const V2 *)(Ap + e * L.pa);
+				ix = (T)1 / c[13].x;
+				iy = (T)1 / c[13].y;
+			}
+		}
+		w -= pw;
+	}
+	__syncthreads();
+	T xe = (T)0, xd = (T)0;
+#pragma unroll 1
+	for (int sw = 0; sw < nsweeps; sw++) {
+		halo_wrap_block<T>(L, xs, 1 + hx + hxy, hx, hxy);
+#pragma unroll 1
+		for (int p = 0; p < 4; p++) lds_pair_step<T, NT>(c, rv, ix, iy, xs + lq, hx, hxy, my == p && live, two, xe, xd);
+	}
+	if (live) {
+		x[at] = xe;
+		if (two) x[at + 1] = xd;
+	}
+}
+
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void k_gs_pairs(LevelView L, const T *__restrict__ A, T *__restrict__ x,
+						 const T *__restrict__ r, int nsweeps) {
+	extern __shared__ __align__(16) char smem_[];
+	gs_lds_pairs<T, NT>(L, A, x, r, nsweeps, (T *)smem_);
+}
+
 template <typename T>
 __global__ __launch_bounds__(1024) void k_gs_small_lds(LevelView L, const T *__restrict__ A, T *__restrict__ x,
 						       const T *__restrict__ r, int nsweeps, int mode, int exact) {
@@ -2024,7 +2139,12 @@ __global__ __launch_bounds__(1024) void k_gs_small(LevelView L, const T *__restr
 template <typename T>
 void launch_gs_small(hipStream_t s, const LevelView &L, const T *A, T *x, const T *r, int nsweeps, int mode, int exact) {
 	const long long lds = small_lds_bytes(L, (int)sizeof(T));
-	if (lds <= kSmallLdsBytes)
+	const int nt = exact || mode || nsweeps < 1 ? 0 : pair_threads(L, (int)sizeof(T));
+	if (nt == 512)
+		hipLaunchKernelGGL((k_gs_pairs<T, 512>), dim3(1), dim3(512), (unsigned)pair_lds_bytes(L, (int)sizeof(T)), s, L, A, x, r, nsweeps);
+	else if (nt == 768)
+		hipLaunchKernelGGL((k_gs_pairs<T, 768>), dim3(1), dim3(768), (unsigned)pair_lds_bytes(L, (int)sizeof(T)), s, L, A, x, r, nsweeps);
+	else if (lds <= kSmallLdsBytes)
 		hipLaunchKernelGGL(k_gs_small_lds<T>, dim3(1), dim3(1024), (unsigned)lds, s, L, A, x, r, nsweeps, mode, exact);
 	else
 		hipLaunchKernelGGL(k_gs_small<T>, dim3(1), dim3(1024), 0, s, L, A, x, r, nsweeps, mode, exact);
@@ -3790,13 +3910,19 @@ __global__ __launch_bounds__(256) void kb_gs_pair(const SlotDev *__restrict__ sl
 	}
 }
 
+// 768 threads: the most k_gs_pairs takes; a level with point pairs in more
+// wavefronts takes the one-point-a-thread form where it has a thread a point.
+constexpr int kBatchSmall = 768;
 template <typename T>
-__global__ __launch_bounds__(1024) void kb_gs_small(const SlotDev *__restrict__ slots, WorkList wl, int level, int nsweeps) {
-	extern __shared__ char smem_[];
+__global__ __launch_bounds__(kBatchSmall) void kb_gs_small(const SlotDev *__restrict__ slots, WorkList wl, int level,
+							    int nsweeps) {
+	extern __shared__ __align__(16) char smem_[];
 	BATCH_LOOP
 		(void)lu;
 		const LevelView L = S->lv[level];
-		if (small_lds_bytes(L, (int)sizeof(T)) <= kSmallLdsBytes)
+		if (pair_threads(L, (int)sizeof(T)) > 0)
+			gs_lds_pairs<T, kBatchSmall>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), nsweeps, (T *)smem_);
+		else if (small_lds_bytes(L, (int)sizeof(T)) <= kSmallLdsBytes)
 			gs_lds_body<T>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), nsweeps, 0, 0, (T *)smem_);
 		else
 			gs_small_body<T>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), nsweeps, 0, 0);
@@ -3924,7 +4050,7 @@ void launch_b_gs_pair(hipStream_t s, const SlotDev *slots, WorkList wl, int leve
 template <typename T>
 void launch_b_gs_small(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int nsweeps) {
 	if (wl.n <= 0) return;
-	hipLaunchKernelGGL(kb_gs_small<T>, dim3(batch_grid(wl)), dim3(1024), kSmallLdsBytes, s, slots, wl, level, nsweeps);
+	hipLaunchKernelGGL(kb_gs_small<T>, dim3(batch_grid(wl)), dim3(kBatchSmall), kSmallLdsBytes, s, slots, wl, level, nsweeps);
 	HIPCHECK_LAUNCH();
 }
 template <typename T>
