@@ -3845,14 +3845,22 @@ template <typename T> __device__ __forceinline__ T *sA(const SlotDev *S, int l);
 template <typename T> __device__ __forceinline__ T *sx(const SlotDev *S, int l);
 template <typename T> __device__ __forceinline__ T *sr(const SlotDev *S, int l);
 template <typename T> __device__ __forceinline__ T *sres(const SlotDev *S);
-template <> __device__ __forceinline__ double *sA<double>(const SlotDev *S, int l) { return S->A[l]; }
-template <> __device__ __forceinline__ double *sx<double>(const SlotDev *S, int l) { return S->x[l]; }
-template <> __device__ __forceinline__ double *sr<double>(const SlotDev *S, int l) { return S->r[l]; }
-template <> __device__ __forceinline__ double *sres<double>(const SlotDev *S) { return S->res64; }
-template <> __device__ __forceinline__ float *sA<float>(const SlotDev *S, int l) { return S->A32[l]; }
-template <> __device__ __forceinline__ float *sx<float>(const SlotDev *S, int l) { return S->x32[l]; }
-template <> __device__ __forceinline__ float *sr<float>(const SlotDev *S, int l) { return S->r32[l]; }
-template <> __device__ __forceinline__ float *sres<float>(const SlotDev *S) { return S->res32; }
+// A pointer of the slot table, read through the constant address space: the
+// compiler takes a pointer from there to be a global one.  Otherwise it cannot
+// tell (the table is ordinary memory) and issues flat loads, which count as
+// LDS accesses too, so every row step of a row kernel waited for its own loads,
+// nine round trips in place of one.
+template <typename P> __device__ __forceinline__ P *slot_ptr(P *const &field) {
+	return *(P *const __attribute__((address_space(4))) *)&field;
+}
+template <> __device__ __forceinline__ double *sA<double>(const SlotDev *S, int l) { return slot_ptr(S->A[l]); }
+template <> __device__ __forceinline__ double *sx<double>(const SlotDev *S, int l) { return slot_ptr(S->x[l]); }
+template <> __device__ __forceinline__ double *sr<double>(const SlotDev *S, int l) { return slot_ptr(S->r[l]); }
+template <> __device__ __forceinline__ double *sres<double>(const SlotDev *S) { return slot_ptr(S->res64); }
+template <> __device__ __forceinline__ float *sA<float>(const SlotDev *S, int l) { return slot_ptr(S->A32[l]); }
+template <> __device__ __forceinline__ float *sx<float>(const SlotDev *S, int l) { return slot_ptr(S->x32[l]); }
+template <> __device__ __forceinline__ float *sr<float>(const SlotDev *S, int l) { return slot_ptr(S->r32[l]); }
+template <> __device__ __forceinline__ float *sres<float>(const SlotDev *S) { return slot_ptr(S->res32); }
 
 // Decodes a 64x4-point block unit of level view L into the thread's point.
 __device__ __forceinline__ bool pts_unit(const LevelView &L, int lu, int &i, int &j, int &k) {
@@ -3886,19 +3894,50 @@ __device__ __forceinline__ bool cubes_unit(const LevelView &L, int lu, int &ic, 
 	return ic < ncx && jc < ncy;
 }
 
+// A list of up to 64 slots in a wavefront's registers, lane q holding slot q
+// and the end of its units.  The unit's slot is then one ballot; bisection
+// over the list in memory is five or six dependent loads, and on the launches
+// of small levels, a few workgroups long, those were most of the time
+// (16 us a launch where the lone kernel takes 4).
+struct ListLanes {
+	int end, slot;
+	__device__ __forceinline__ ListLanes(const WorkList &wl) : end(0x7fffffff), slot(0) {
+		const int l = __lane_id();
+		if (wl.n <= 64 && l < wl.n) {
+			end = wl.prefix[l + 1];
+			slot = wl.slot[l];
+		}
+	}
+	// unit u's place in the list: its slot, and the number of the slot's
+	// first unit (every lane of the wavefront must be active)
+	__device__ __forceinline__ void find(int u, int &s, int &first) const {
+		const int q = __popcll(__ballot(end <= u));
+		s = __builtin_amdgcn_readlane(slot, q);
+		first = q > 0 ? __builtin_amdgcn_readlane(end, q - 1) : 0;
+	}
+};
+
 // Each workgroup takes one contiguous chunk of the list's units (chunks
-// numbered per XCD, so neighbouring units share an L2), finds the first
-// unit's slot by bisection and then walks forward through the slots.
+// numbered per XCD, so neighbouring units share an L2), and finds each unit's
+// slot (ListLanes), or, on a longer list, the first unit's by bisection and
+// then walks forward through the slots.
 #define BATCH_LOOP                                                                         \
-	const int total_ = wl.prefix[wl.n];                                                \
+	const int total_ = wl.total;                                                       \
 	const int per_ = (total_ + (int)gridDim.x - 1) / (int)gridDim.x;                   \
 	const int u0_ = xcd_block((int)blockIdx.x, (int)gridDim.x) * per_;                 \
 	const int u1_ = min(total_, u0_ + per_);                                           \
-	int q_ = u0_ < u1_ ? __builtin_amdgcn_readfirstlane(wl_find(wl, u0_)) : 0;         \
+	const ListLanes lanes_(wl);                                                        \
+	int q_ = wl.n > 64 && u0_ < u1_ ? __builtin_amdgcn_readfirstlane(wl_find(wl, u0_)) : 0; \
 	for (int u = u0_; u < u1_; u++) {                                                  \
-		while (u >= wl.prefix[q_ + 1]) q_++;                                       \
-		const SlotDev *S = slots + wl.slot[q_];                                    \
-		const int lu = u - wl.prefix[q_];
+		int slot_, first_;                                                         \
+		if (wl.n <= 64) lanes_.find(u, slot_, first_);                             \
+		else {                                                                     \
+			while (u >= wl.prefix[q_ + 1]) q_++;                               \
+			slot_ = wl.slot[q_];                                               \
+			first_ = wl.prefix[q_];                                            \
+		}                                                                          \
+		const SlotDev *S = slots + slot_;                                          \
+		const int lu = u - first_;
 
 template <typename T, bool Z = false>
 __global__ __launch_bounds__(256) void kb_gs_pair(const SlotDev *__restrict__ slots, WorkList wl,
@@ -3945,11 +3984,12 @@ __global__ __launch_bounds__(256) void kb_residual_top(const SlotDev *__restrict
 	BATCH_LOOP
 		const LevelView L = S->lv[0];
 		const int w = __builtin_amdgcn_readfirstlane(lu * 4 + (int)threadIdx.y);
-		const double v2 = to_f32 ? residual_wave<double, float>(L, S->A[0], S->x[0], S->r[0], S->r32[0],
-									 S->top_zero ? (float *)nullptr : S->x32[0], w)
-					 : residual_wave<double, double>(L, S->A[0], S->x[0], S->r[0], (double *)nullptr, (double *)nullptr, w);
+		const double *A = sA<double>(S, 0), *x = sx<double>(S, 0), *r = sr<double>(S, 0);
+		const double v2 = to_f32 ? residual_wave<double, float>(L, A, x, r, sr<float>(S, 0),
+									 S->top_zero ? (float *)nullptr : sx<float>(S, 0), w)
+					 : residual_wave<double, double>(L, A, x, r, (double *)nullptr, (double *)nullptr, w);
 		const double sblk = block_sum_256(v2);
-		if (threadIdx.x == 0 && threadIdx.y == 0) S->partial[lu] = sblk;
+		if (threadIdx.x == 0 && threadIdx.y == 0) slot_ptr(S->partial)[lu] = sblk;
 		__syncthreads();
 	}
 }
@@ -3961,14 +4001,14 @@ __global__ __launch_bounds__(1024) void kb_reduce(const SlotDev *__restrict__ sl
 		const LevelView L = S->lv[0];
 		const int n = residual_blocks(L, 8);
 		double s = 0.0;
-		for (int t = threadIdx.x; t < n; t += 1024) s = s + S->partial[t];
+		for (int t = threadIdx.x; t < n; t += 1024) s = s + slot_ptr(S->partial)[t];
 		red[threadIdx.x] = s;
 		__syncthreads();
 		for (int w = 512; w > 0; w >>= 1) {
 			if ((int)threadIdx.x < w) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + w];
 			__syncthreads();
 		}
-		if (threadIdx.x == 0) norms[wl.slot[q_]] = red[0];
+		if (threadIdx.x == 0) norms[slot_] = red[0];
 		__syncthreads();
 	}
 }
@@ -4008,7 +4048,7 @@ template <typename T>
 __global__ __launch_bounds__(1024) void kb_lu_solve(const SlotDev *__restrict__ slots, WorkList wl, int level) {
 	BATCH_LOOP
 		(void)lu;
-		lu_solve_body<T>(S->lv[level], S->lu_n, S->LU, S->ipiv, sr<T>(S, level), sx<T>(S, level));
+		lu_solve_body<T>(S->lv[level], S->lu_n, slot_ptr(S->LU), slot_ptr(S->ipiv), sr<T>(S, level), sx<T>(S, level));
 		__syncthreads();
 	}
 }
@@ -4019,7 +4059,8 @@ __global__ __launch_bounds__(256) void kb_add_x(const SlotDev *__restrict__ slot
 		int i, j, k;
 		if (flat_unit(L, lu, i, j, k)) {
 			const long long p = idx3(L, i, j, k);
-			S->x[0][p] = S->x[0][p] + (double)S->x32[0][p];
+			double *x = sx<double>(S, 0);
+			x[p] = x[p] + (double)sx<float>(S, 0)[p];
 		}
 	}
 }
