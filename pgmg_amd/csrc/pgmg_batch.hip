@@ -156,6 +156,7 @@ struct pgmg_batch {
 	std::vector<int> h_plan;
 	int list_stride = 0;
 	std::vector<int> list_n;  // slots per list
+	std::vector<long long> level_bytes;  // coefficients of a level of all slots
 	bool plan_dirty = true;
 	double *d_norms = nullptr, *h_norms = nullptr;
 	double *d_aux = nullptr, *h_aux = nullptr;  // per slot: source norm, LU flag
@@ -178,6 +179,15 @@ void drop_graph(pgmg_batch *b) {
 	b->plan_steps = 0;
 }
 
+// A level's coefficients, of all its slots together, that the launches read
+// with plain loads, to find them in the memory-side cache (256 MB) in the next
+// sweep; larger levels are streamed, as when side by side they would push
+// each other out.  (A small level of a few slots streamed from HBM takes
+// twice as long a launch.)  16 problems of 33 to 129 points an axis: 857 ms
+// all streamed, 747 with 32 MB, 736 with 64, 722 with 128 and 256, 732 with
+// everything cached.
+const long long kCacheBytes = 128LL << 20;
+
 int list_index(int level, int kind) { return L_TOP_COUNT + level * L_PER_LEVEL + kind; }
 int n_lists() { return L_TOP_COUNT + kBatchMaxLevels * L_PER_LEVEL; }
 
@@ -187,6 +197,7 @@ WorkList wlist(pgmg_batch *b, int li) {
 	w.prefix = w.slot + b->max_slots;
 	w.n = b->list_n[li];
 	w.total = b->h_plan[(size_t)li * b->list_stride + b->max_slots + w.n];
+	w.cache = li >= L_TOP_COUNT && b->level_bytes[(li - L_TOP_COUNT) / L_PER_LEVEL] <= kCacheBytes;
 	return w;
 }
 
@@ -202,6 +213,7 @@ void plan_add(pgmg_batch *b, int li, int slot, int units) {
 int build_plan(pgmg_batch *b) {
 	const int el = b->mixed ? 4 : 8;  // the cycle's arithmetic
 	std::fill(b->list_n.begin(), b->list_n.end(), 0);
+	b->level_bytes.assign(kBatchMaxLevels, 0);
 	for (int li = 0; li < n_lists(); li++) b->h_plan[(size_t)li * b->list_stride + b->max_slots] = 0;
 	b->max_nl = 0;
 	for (int s = 0; s < b->max_slots; s++) {
@@ -214,6 +226,7 @@ int build_plan(pgmg_batch *b) {
 		plan_add(b, L_TOP_PTS, s, batch_units(BK_FLAT, D.lv[0], 8));
 		for (int l = 0; l < S.nl; l++) {
 			const LevelView &L = D.lv[l];
+			b->level_bytes[l] += 27LL * el * L.m * L.n * L.o;
 			if (l < S.nl - 1) {
 				// as the lone hierarchy's forward colour sweeps
 				if (batch_level_small(L, el))
@@ -235,8 +248,14 @@ int build_plan(pgmg_batch *b) {
 	return PGMG_OK;
 }
 
-int chunk_of(pgmg_batch *b, int cls) {
-	return b->tune.done ? b->tune.best[cls] : kChunks[b->tune.step % kNumChunks];
+// A launch keeps at least kMinGroups workgroups (four to a CU) where its units
+// allow: with fewer, units that could run side by side follow one another in a
+// workgroup (a trial of 8 units a workgroup took 65 us on levels of 40 units
+// that take 12 one by one).
+const int kMinGroups = 1024;
+int chunk_of(pgmg_batch *b, int cls, int units) {
+	const int c = b->tune.done ? b->tune.best[cls] : kChunks[b->tune.step % kNumChunks];
+	return std::max(1, std::min(c, units / kMinGroups));
 }
 
 // Runs launch(chunk) for class cls; during the trial steps it is bracketed
@@ -244,7 +263,7 @@ int chunk_of(pgmg_batch *b, int cls) {
 template <typename F>
 void tuned(pgmg_batch *b, int cls, const WorkList &wl, F launch) {
 	if (wl.n <= 0) return;
-	const int c = chunk_of(b, cls);
+	const int c = chunk_of(b, cls, wl.total);
 	TileTuner &t = b->tune;
 	if (t.done) { launch(c); return; }
 	if (t.used + 2 > t.pool.size()) {

@@ -206,6 +206,8 @@ struct WorkList {
 	const int *prefix;
 	int n;
 	int total;  // prefix[n], known to the host: the launch's grid size
+	int cache;  // 1: the colour-pair and residual kernels read the slots'
+	            // coefficients with plain loads (LevelView::cache_coef)
 };
 // Unit kinds: the colour-pair row groups of a level, one unit per slot,
 // residual row groups, 64x4-point blocks of a level, 64x4 blocks of its

@@ -3943,7 +3943,8 @@ template <typename T, bool Z = false>
 __global__ __launch_bounds__(256) void kb_gs_pair(const SlotDev *__restrict__ slots, WorkList wl,
 								   int level, int cj, int ck) {
 	BATCH_LOOP
-		const LevelView L = S->lv[level];
+		LevelView L = S->lv[level];
+		L.cache_coef = (short)wl.cache;
 		gs_wave<T, Z, false>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), cj, ck,
 			      __builtin_amdgcn_readfirstlane(lu * 4 + (int)threadIdx.y));
 	}
@@ -3972,7 +3973,8 @@ __global__ __launch_bounds__(kBatchSmall) void kb_gs_small(const SlotDev *__rest
 template <typename T>
 __global__ __launch_bounds__(256) void kb_residual(const SlotDev *__restrict__ slots, WorkList wl, int level) {
 	BATCH_LOOP
-		const LevelView L = S->lv[level];
+		LevelView L = S->lv[level];
+		L.cache_coef = (short)wl.cache;
 		(void)residual_wave<T, T>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), sres<T>(S), (T *)nullptr,
 					  __builtin_amdgcn_readfirstlane(lu * 4 + (int)threadIdx.y));
 	}
