@@ -112,7 +112,9 @@ int shape_dims(int m, int n, int o, int *dims) {
 
 // Lists of the plan.
 enum { L_PAIR0 = 0, L_PAIR1, L_PAIR2, L_PAIR3, L_SMALL, L_RES, L_RESTRICT, L_INTERP, L_LU, L_GS24, L_PER_LEVEL };
-enum { L_TOP_ROWS = 0, L_TOP_ONE, L_TOP_PTS, L_TOP_COUNT };
+// L_X_*: level-0 lists of the slots whose operator is a 7-point cross
+// (LevelView::cross), which take kernels of their own there.
+enum { L_TOP_ROWS = 0, L_X_TOP_ROWS, L_TOP_ONE, L_TOP_PTS, L_X_PAIR0, L_X_PAIR1, L_X_PAIR2, L_X_PAIR3, L_X_RES, L_TOP_COUNT };
 
 // Tile shapes of the batched launches: work units per workgroup, one choice
 // per launch class, measured on the batch's own first steps.  Trial t
@@ -197,7 +199,9 @@ WorkList wlist(pgmg_batch *b, int li) {
 	w.prefix = w.slot + b->max_slots;
 	w.n = b->list_n[li];
 	w.total = b->h_plan[(size_t)li * b->list_stride + b->max_slots + w.n];
-	w.cache = li >= L_TOP_COUNT && b->level_bytes[(li - L_TOP_COUNT) / L_PER_LEVEL] <= kCacheBytes;
+	const bool level0 = li >= L_X_PAIR0 && li < L_TOP_COUNT;
+	w.cache = (level0 && b->level_bytes[0] <= kCacheBytes) ||
+		  (li >= L_TOP_COUNT && b->level_bytes[(li - L_TOP_COUNT) / L_PER_LEVEL] <= kCacheBytes);
 	return w;
 }
 
@@ -221,18 +225,20 @@ int build_plan(pgmg_batch *b) {
 		if (S.state != ST_ACTIVE) continue;
 		const SlotDev &D = S.dev;
 		b->max_nl = std::max(b->max_nl, S.nl);
-		plan_add(b, L_TOP_ROWS, s, batch_units(BK_ROWS, D.lv[0], 8));
+		plan_add(b, D.lv[0].cross ? L_X_TOP_ROWS : L_TOP_ROWS, s, batch_units(BK_ROWS, D.lv[0], 8));
 		plan_add(b, L_TOP_ONE, s, 1);
 		plan_add(b, L_TOP_PTS, s, batch_units(BK_FLAT, D.lv[0], 8));
 		for (int l = 0; l < S.nl; l++) {
 			const LevelView &L = D.lv[l];
-			b->level_bytes[l] += 27LL * el * L.m * L.n * L.o;
+			const bool x = L.cross != 0;  // level 0 only
+			b->level_bytes[l] += (x ? 7LL : 27LL) * el * L.m * L.n * L.o;
 			if (l < S.nl - 1) {
 				// as the lone hierarchy's forward colour sweeps
 				if (batch_level_small(L, el))
 					plan_add(b, list_index(l, L_SMALL), s, 1);
-				else for (int q = 0; q < 4; q++) plan_add(b, list_index(l, L_PAIR0 + q), s, batch_units(BK_PAIR0 + q, L, el));
-				plan_add(b, list_index(l, L_RES), s, batch_units(BK_ROWS, L, el));
+				else for (int q = 0; q < 4; q++)
+					plan_add(b, x ? L_X_PAIR0 + q : list_index(l, L_PAIR0 + q), s, batch_units(BK_PAIR0 + q, L, el));
+				plan_add(b, x ? L_X_RES : list_index(l, L_RES), s, batch_units(BK_ROWS, L, el));
 				plan_add(b, list_index(l + 1, L_RESTRICT), s, batch_restrict_units(L, D.lv[l + 1]));
 				plan_add(b, list_index(l + 1, L_INTERP), s, batch_units(BK_CUBES, L, el));
 			} else if (D.lu_active) {
@@ -319,10 +325,12 @@ void batched_gs(pgmg_batch *b, int l, int sweeps, bool from_zero = false) {
 	if (sweeps <= 0) return;
 	for (int s = 0; s < sweeps; s++)
 		for (int q = 0; q < 4; q++) {
+			const bool fz = from_zero && s == 0;
 			const WorkList wl = wlist(b, list_index(l, L_PAIR0 + q));
-			tuned(b, TC_PAIR, wl, [&](int c) {
-				launch_b_gs_pair<T>(b->stream, b->d_slots, wl, l, q, from_zero && s == 0, c);
-			});
+			tuned(b, TC_PAIR, wl, [&](int c) { launch_b_gs_pair<T>(b->stream, b->d_slots, wl, l, q, fz, c); });
+			if (l > 0) continue;
+			const WorkList wx = wlist(b, L_X_PAIR0 + q);
+			tuned(b, TC_PAIR, wx, [&](int c) { launch_b_gs_pair<T>(b->stream, b->d_slots, wx, l, q, fz, c, true); });
 		}
 	launch_b_gs_small<T>(b->stream, b->d_slots, wlist(b, list_index(l, L_SMALL)), l, sweeps);
 }
@@ -335,6 +343,10 @@ void batched_cycle(pgmg_batch *b) {
 		batched_gs<T>(b, l, b->opts.v_down + l, b->mixed && l == 0);
 		const WorkList wr = wlist(b, list_index(l, L_RES));
 		tuned(b, TC_RES, wr, [&](int c) { launch_b_residual<T>(b->stream, b->d_slots, wr, l, c); });
+		if (l == 0) {
+			const WorkList wx = wlist(b, L_X_RES);
+			tuned(b, TC_RES, wx, [&](int c) { launch_b_residual<T>(b->stream, b->d_slots, wx, l, c, true); });
+		}
 		if (l + 1 < kBatchMaxLevels) {
 			const WorkList wt = wlist(b, list_index(l + 1, L_RESTRICT));
 			tuned(b, TC_RESTRICT, wt, [&](int c) { launch_b_restrict<T>(b->stream, b->d_slots, wt, l + 1, c); });
@@ -447,19 +459,26 @@ int slot_setup(pgmg_batch *b, int s, const pgmg_dims *d, int family, uint64_t se
 	hipStream_t st = b->setup;
 	launch_fill<double>(st, (double *)(b->arena.base + S.off), (long long)(S.bytes / 8), 0.0);
 	if (family) {
+		D.lv[0].cross = family != PGMG_FAM_Q1_ANISO && cross_pays(D.lv[0]);
 		launch_generate(st, D.lv[0], family, seed, D.A[0], D.r[0]);
 	} else {
 		// host operator and source: staged through the level-0 x and r32
 		// arrays is not possible for every size, so copy synchronously.
 		const long long N0 = (long long)D.lv[0].m * D.lv[0].n * D.lv[0].o;
 		double *stage = nullptr;
-		BHIP(hipMalloc(&stage, sizeof(double) * 27 * (size_t)N0));
+		// and, after the operator, whether it has an entry outside the
+		// 7-point cross
+		BHIP(hipMalloc(&stage, sizeof(double) * (27 * (size_t)N0 + 1)));
+		int *dense = (int *)(stage + 27 * N0);
+		launch_fill<int>(st, dense, 1, 0);
 		BHIP(hipMemcpyAsync(stage, A27, sizeof(double) * 27 * N0, hipMemcpyHostToDevice, st));
-		launch_pack_op(st, D.lv[0], stage, D.A[0], 0, N0);
+		launch_pack_op(st, D.lv[0], stage, D.A[0], 0, N0, dense);
+		BHIP(hipMemcpyAsync(b->h_aux + 2 * s + 1, dense, sizeof(int), hipMemcpyDeviceToHost, st));
 		BHIP(hipMemcpyAsync(stage, rhs, sizeof(double) * N0, hipMemcpyHostToDevice, st));
 		launch_pack_vec(st, D.lv[0], stage, D.r[0], 0, N0);
 		BHIP(hipStreamSynchronize(st));
 		hipFree(stage);
+		D.lv[0].cross = *(const int *)(b->h_aux + 2 * s + 1) == 0 && cross_pays(D.lv[0]);
 	}
 	for (int l = 1; l < S.nl; l++) launch_rat(st, D.lv[l - 1], D.lv[l], D.A[l - 1], D.A[l]);
 	if (S.want_lu) {
@@ -620,11 +639,13 @@ int pgmg_batch_step(pgmg_batch *b, int *active, int *finished) {
 	}
 	if (b->plan_dirty) { rc = build_plan(b); if (rc) return rc; }
 	int nfin = 0, nact = 0;
-	if (b->list_n[L_TOP_ROWS] > 0) {
+	if (b->list_n[L_TOP_ONE] > 0) {
 		// residual of the current iterate: convergence test, and the FP32
 		// defect for the mixed-precision cycle
 		const WorkList wtop = wlist(b, L_TOP_ROWS);
 		tuned(b, TC_RESTOP, wtop, [&](int c) { launch_b_residual_top(b->stream, b->d_slots, wtop, b->mixed, c); });
+		const WorkList wxtop = wlist(b, L_X_TOP_ROWS);
+		tuned(b, TC_RESTOP, wxtop, [&](int c) { launch_b_residual_top(b->stream, b->d_slots, wxtop, b->mixed, c, true); });
 		launch_b_reduce(b->stream, b->d_slots, wlist(b, L_TOP_ONE), b->d_norms);
 		BHIP(hipMemcpyAsync(b->h_norms, b->d_norms, sizeof(double) * b->max_slots, hipMemcpyDeviceToHost, b->stream));
 		BHIP(hipStreamSynchronize(b->stream));
@@ -639,7 +660,7 @@ int pgmg_batch_step(pgmg_batch *b, int *active, int *finished) {
 			else if (std::isnan(e) || S.cycles >= S.max_cycles) { S.state = ST_FAILED; nfin++; }
 		}
 		if (nfin) { rc = build_plan(b); if (rc) return rc; }
-		if (b->list_n[L_TOP_ROWS] > 0) {
+		if (b->list_n[L_TOP_ONE] > 0) {
 			rc = run_cycle(b);
 			if (rc) return rc;
 			BHIP(hipGetLastError());

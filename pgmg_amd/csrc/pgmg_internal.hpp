@@ -226,11 +226,13 @@ int batch_restrict_units(const LevelView &F, const LevelView &C);
 // depend on it, so every chunk gives the same results.
 // from_zero (FP32): the first sweep of level 0 of a mixed correction (slots
 // with top_zero set; the others are in the small-level list).
+// cross: the slots of the list are 7-point crosses on the level.
 template <typename T> void launch_b_gs_pair(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int pair,
-					    bool from_zero = false, int chunk = 1);
+					    bool from_zero = false, int chunk = 1, bool cross = false);
 template <typename T> void launch_b_gs_small(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int nsweeps);
-template <typename T> void launch_b_residual(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk = 1);
-void launch_b_residual_top(hipStream_t s, const SlotDev *slots, WorkList wl, bool to_f32, int chunk = 1);
+template <typename T> void launch_b_residual(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk = 1,
+					     bool cross = false);
+void launch_b_residual_top(hipStream_t s, const SlotDev *slots, WorkList wl, bool to_f32, int chunk = 1, bool cross = false);
 void launch_b_reduce(hipStream_t s, const SlotDev *slots, WorkList wl, double *norms);
 template <typename T> void launch_b_restrict(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk = 1);
 template <typename T> void launch_b_interp(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk = 1);

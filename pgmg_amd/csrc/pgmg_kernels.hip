@@ -3939,13 +3939,15 @@ struct ListLanes {
 		const SlotDev *S = slots + slot_;                                          \
 		const int lu = u - first_;
 
-template <typename T, bool Z = false>
+// X: the list's slots are 7-point crosses on this level (level 0); see
+// coef_or_zero.
+template <typename T, bool Z, bool X>
 __global__ __launch_bounds__(256) void kb_gs_pair(const SlotDev *__restrict__ slots, WorkList wl,
 								   int level, int cj, int ck) {
 	BATCH_LOOP
 		LevelView L = S->lv[level];
 		L.cache_coef = (short)wl.cache;
-		gs_wave<T, Z, false>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), cj, ck,
+		gs_wave<T, Z, false, X>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), cj, ck,
 			      __builtin_amdgcn_readfirstlane(lu * 4 + (int)threadIdx.y));
 	}
 }
@@ -3970,26 +3972,27 @@ __global__ __launch_bounds__(kBatchSmall) void kb_gs_small(const SlotDev *__rest
 	}
 }
 
-template <typename T>
+template <typename T, bool X>
 __global__ __launch_bounds__(256) void kb_residual(const SlotDev *__restrict__ slots, WorkList wl, int level) {
 	BATCH_LOOP
 		LevelView L = S->lv[level];
 		L.cache_coef = (short)wl.cache;
-		(void)residual_wave<T, T>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), sres<T>(S), (T *)nullptr,
+		(void)residual_wave<T, T, X>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), sres<T>(S), (T *)nullptr,
 					  __builtin_amdgcn_readfirstlane(lu * 4 + (int)threadIdx.y));
 	}
 }
 
 // Top-level FP64 residual with per-slot block sums; optionally the residual
 // rounded to FP32 into the slot's level-0 r32 (the defect-correction source).
+template <bool X>
 __global__ __launch_bounds__(256) void kb_residual_top(const SlotDev *__restrict__ slots, WorkList wl, int to_f32) {
 	BATCH_LOOP
 		const LevelView L = S->lv[0];
 		const int w = __builtin_amdgcn_readfirstlane(lu * 4 + (int)threadIdx.y);
 		const double *A = sA<double>(S, 0), *x = sx<double>(S, 0), *r = sr<double>(S, 0);
-		const double v2 = to_f32 ? residual_wave<double, float>(L, A, x, r, sr<float>(S, 0),
+		const double v2 = to_f32 ? residual_wave<double, float, X>(L, A, x, r, sr<float>(S, 0),
 									 S->top_zero ? (float *)nullptr : sx<float>(S, 0), w)
-					 : residual_wave<double, double>(L, A, x, r, (double *)nullptr, (double *)nullptr, w);
+					 : residual_wave<double, double, X>(L, A, x, r, (double *)nullptr, (double *)nullptr, w);
 		const double sblk = block_sum_256(v2);
 		if (threadIdx.x == 0 && threadIdx.y == 0) slot_ptr(S->partial)[lu] = sblk;
 		__syncthreads();
@@ -4076,18 +4079,21 @@ static unsigned batch_grid(const WorkList &wl, int chunk = 1) {
 }
 
 template <typename T>
-void launch_b_gs_pair(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int pair, bool from_zero, int chunk) {
+void launch_b_gs_pair(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int pair, bool from_zero, int chunk,
+		      bool cross) {
 	if (wl.n <= 0) return;
+	const dim3 grid(batch_grid(wl, chunk)), block(64, 4);
+	const int cj = pair & 1, ck = (pair >> 1) & 1;
 	if constexpr (sizeof(T) == 4) {
 		if (from_zero) {
-			hipLaunchKernelGGL((kb_gs_pair<T, true>), dim3(batch_grid(wl, chunk)), dim3(64, 4), 0, s, slots, wl, level, pair & 1,
-					   (pair >> 1) & 1);
+			if (cross) hipLaunchKernelGGL((kb_gs_pair<T, true, true>), grid, block, 0, s, slots, wl, level, cj, ck);
+			else hipLaunchKernelGGL((kb_gs_pair<T, true, false>), grid, block, 0, s, slots, wl, level, cj, ck);
 			HIPCHECK_LAUNCH();
 			return;
 		}
 	}
-	hipLaunchKernelGGL((kb_gs_pair<T, false>), dim3(batch_grid(wl, chunk)), dim3(64, 4), 0, s, slots, wl, level, pair & 1,
-			   (pair >> 1) & 1);
+	if (cross) hipLaunchKernelGGL((kb_gs_pair<T, false, true>), grid, block, 0, s, slots, wl, level, cj, ck);
+	else hipLaunchKernelGGL((kb_gs_pair<T, false, false>), grid, block, 0, s, slots, wl, level, cj, ck);
 	HIPCHECK_LAUNCH();
 }
 template <typename T>
@@ -4097,14 +4103,18 @@ void launch_b_gs_small(hipStream_t s, const SlotDev *slots, WorkList wl, int lev
 	HIPCHECK_LAUNCH();
 }
 template <typename T>
-void launch_b_residual(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk) {
+void launch_b_residual(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk, bool cross) {
 	if (wl.n <= 0) return;
-	hipLaunchKernelGGL(kb_residual<T>, dim3(batch_grid(wl, chunk)), dim3(64, 4), 0, s, slots, wl, level);
+	const dim3 grid(batch_grid(wl, chunk)), block(64, 4);
+	if (cross) hipLaunchKernelGGL((kb_residual<T, true>), grid, block, 0, s, slots, wl, level);
+	else hipLaunchKernelGGL((kb_residual<T, false>), grid, block, 0, s, slots, wl, level);
 	HIPCHECK_LAUNCH();
 }
-void launch_b_residual_top(hipStream_t s, const SlotDev *slots, WorkList wl, bool to_f32, int chunk) {
+void launch_b_residual_top(hipStream_t s, const SlotDev *slots, WorkList wl, bool to_f32, int chunk, bool cross) {
 	if (wl.n <= 0) return;
-	hipLaunchKernelGGL(kb_residual_top, dim3(batch_grid(wl, chunk)), dim3(64, 4), 0, s, slots, wl, to_f32 ? 1 : 0);
+	const dim3 grid(batch_grid(wl, chunk)), block(64, 4);
+	if (cross) hipLaunchKernelGGL(kb_residual_top<true>, grid, block, 0, s, slots, wl, to_f32 ? 1 : 0);
+	else hipLaunchKernelGGL(kb_residual_top<false>, grid, block, 0, s, slots, wl, to_f32 ? 1 : 0);
 	HIPCHECK_LAUNCH();
 }
 void launch_b_reduce(hipStream_t s, const SlotDev *slots, WorkList wl, double *norms) {
@@ -4156,9 +4166,9 @@ void launch_b_add_x(hipStream_t s, const SlotDev *slots, WorkList wl, int chunk)
 	template bool gs_tile_ok<T>(const LevelView &); \
 	template void launch_lu_solve<T>(hipStream_t, const LevelView &, int, const double *, const int *, const T *, T *); \
 	template void launch_fill<T>(hipStream_t, T *, long long, T); \
-	template void launch_b_gs_pair<T>(hipStream_t, const SlotDev *, WorkList, int, int, bool, int); \
+	template void launch_b_gs_pair<T>(hipStream_t, const SlotDev *, WorkList, int, int, bool, int, bool); \
 	template void launch_b_gs_small<T>(hipStream_t, const SlotDev *, WorkList, int, int); \
-	template void launch_b_residual<T>(hipStream_t, const SlotDev *, WorkList, int, int); \
+	template void launch_b_residual<T>(hipStream_t, const SlotDev *, WorkList, int, int, bool); \
 	template void launch_b_restrict<T>(hipStream_t, const SlotDev *, WorkList, int, int); \
 	template void launch_b_interp<T>(hipStream_t, const SlotDev *, WorkList, int, int); \
 	template void launch_b_lu_solve<T>(hipStream_t, const SlotDev *, WorkList, int);

@@ -80,3 +80,27 @@ def test_operator_replaced_by_a_denser_one():
             mg.set_rhs(b)
             mg.v_cycle()
             assert np.array_equal(h.get_x(), mg.get_x(0))
+
+
+@pytest.mark.parametrize("precision", [P.PREC_FP64, P.PREC_MIXED])
+def test_batch_of_crosses_and_others_equals_alone(precision):
+    dims = [(50, 37, 40), (129, 29, 19), (33, 50, 41), (20, 17, 30), (262, 15, 17), (50, 37, 40)]
+    fams = [P.FAM_FACE7_UNIFORM, P.FAM_FACE7_LOGUNI, P.FAM_Q1_ANISO, P.FAM_FACE7_UNIFORM, P.FAM_FACE7_UNIFORM, P.FAM_Q1_ANISO]
+
+    def alone(m, n, o, fam, seed):
+        with P.Hierarchy(m, n, o, precision=precision) as h:
+            h.generate_problem(fam, seed)
+            h.compute_rats()
+            c, _ = h.solve(1e-7, 12, check=False)
+            return c, h.get_x()
+
+    with P.Batch(1 << 31, max_slots=16, precision=precision) as batch:
+        slots = [batch.admit(*d, f, 60 + q, 1e-7, 12) for q, (d, f) in enumerate(zip(dims, fams))]
+        slots += [batch.admit_operator(O.gen_operator(f, 60 + q, *d), O.gen_rhs(60 + q, *d), 1e-7, 12)
+                  for q, (d, f) in enumerate(zip(dims, fams))]
+        batch.run()
+        for q, (d, f) in enumerate(zip(dims, fams)):
+            c, x = alone(*d, f, 60 + q)
+            for s in (slots[q], slots[q + len(dims)]):
+                assert batch.status(s)[1] == c, (d, f)
+                assert np.array_equal(batch.get_x(s), x), (d, f)
