@@ -95,6 +95,11 @@ struct SlotHost {
 	double bn = 0, rel = 1;
 	bool want_lu = false;
 	uint64_t seq = 0;  // admission order
+	// levels that may sweep a tile a workgroup: tiles (0: not), the larger
+	// workgroup, LDS
+	int tiles[kBatchMaxLevels] = {};
+	bool tile_big[kBatchMaxLevels] = {};
+	size_t tile_lds[kBatchMaxLevels] = {};
 	hipEvent_t ready = nullptr;
 	SlotDev dev;
 };
@@ -111,7 +116,8 @@ int shape_dims(int m, int n, int o, int *dims) {
 }
 
 // Lists of the plan.
-enum { L_PAIR0 = 0, L_PAIR1, L_PAIR2, L_PAIR3, L_SMALL, L_RES, L_RESTRICT, L_INTERP, L_LU, L_GS24, L_PER_LEVEL };
+enum { L_PAIR0 = 0, L_PAIR1, L_PAIR2, L_PAIR3, L_SMALL, L_RES, L_RESTRICT, L_INTERP, L_LU, L_GS24, L_TILE,
+       L_TILE_BIG, L_INTERP_T, L_PER_LEVEL };
 // L_X_*: level-0 lists of the slots whose operator is a 7-point cross
 // (LevelView::cross), which take kernels of their own there.
 enum { L_TOP_ROWS = 0, L_X_TOP_ROWS, L_TOP_ONE, L_TOP_PTS, L_X_PAIR0, L_X_PAIR1, L_X_PAIR2, L_X_PAIR3, L_X_RES, L_TOP_COUNT };
@@ -159,6 +165,7 @@ struct pgmg_batch {
 	int list_stride = 0;
 	std::vector<int> list_n;  // slots per list
 	std::vector<long long> level_bytes;  // coefficients of a level of all slots
+	size_t tile_lds[kBatchMaxLevels][2] = {};  // LDS of a level's L_TILE, L_TILE_BIG launches
 	bool plan_dirty = true;
 	double *d_norms = nullptr, *h_norms = nullptr;
 	double *d_aux = nullptr, *h_aux = nullptr;  // per slot: source norm, LU flag
@@ -214,8 +221,19 @@ void plan_add(pgmg_batch *b, int li, int slot, int units) {
 	n++;
 }
 
+// Most tiles a level's sweeps run as tile launches (launch_b_gs_tile), all
+// its slots together; with more, the colour-pair launches fill the chip.  16
+// problems of 33 to 129 points an axis: 562 ms without tiles, 504 with at most
+// 256, 483 with 512, 453 with 1024, 498 with 1536 and more.
+const long long kMaxTiles = 1024;
+
 int build_plan(pgmg_batch *b) {
 	const int el = b->mixed ? 4 : 8;  // the cycle's arithmetic
+	long long tiles[kBatchMaxLevels] = {};
+	for (const SlotHost &S : b->slots)
+		if (S.state == ST_ACTIVE)
+			for (int l = 0; l < S.nl; l++) tiles[l] += S.tiles[l];
+	memset(b->tile_lds, 0, sizeof b->tile_lds);
 	std::fill(b->list_n.begin(), b->list_n.end(), 0);
 	b->level_bytes.assign(kBatchMaxLevels, 0);
 	for (int li = 0; li < n_lists(); li++) b->h_plan[(size_t)li * b->list_stride + b->max_slots] = 0;
@@ -234,13 +252,21 @@ int build_plan(pgmg_batch *b) {
 			b->level_bytes[l] += (x ? 7LL : 27LL) * el * L.m * L.n * L.o;
 			if (l < S.nl - 1) {
 				// as the lone hierarchy's forward colour sweeps
+				const bool tile = S.tiles[l] > 0 && tiles[l] <= kMaxTiles;
 				if (batch_level_small(L, el))
 					plan_add(b, list_index(l, L_SMALL), s, 1);
-				else for (int q = 0; q < 4; q++)
+				else if (tile) {
+					const int big = S.tile_big[l] ? 1 : 0;
+					plan_add(b, list_index(l, L_TILE + big), s, S.tiles[l]);
+					b->tile_lds[l][big] = std::max(b->tile_lds[l][big], S.tile_lds[l]);
+				} else for (int q = 0; q < 4; q++)
 					plan_add(b, x ? L_X_PAIR0 + q : list_index(l, L_PAIR0 + q), s, batch_units(BK_PAIR0 + q, L, el));
 				plan_add(b, x ? L_X_RES : list_index(l, L_RES), s, batch_units(BK_ROWS, L, el));
 				plan_add(b, list_index(l + 1, L_RESTRICT), s, batch_restrict_units(L, D.lv[l + 1]));
-				plan_add(b, list_index(l + 1, L_INTERP), s, batch_units(BK_CUBES, L, el));
+				// an odd number of tile sweeps follows the interpolation from
+				// the residual scratch, to end in x
+				plan_add(b, list_index(l + 1, tile && ((b->opts.v_up + l) & 1) ? L_INTERP_T : L_INTERP), s,
+					 batch_units(BK_CUBES, L, el));
 			} else if (D.lu_active) {
 				plan_add(b, list_index(l, L_LU), s, 1);
 			} else {
@@ -318,11 +344,18 @@ void tune_collect(pgmg_batch *b) {
 	t.done = true;
 }
 
-// from_zero: level 0 of the mixed correction, whose pair-list slots did not
-// clear x32 (top_zero); the first sweep reads none of it.
+// from_zero: level 0 of the mixed correction, whose pair- and tile-list slots
+// did not clear x32 (top_zero); the first sweep reads none of it.  down: the
+// sweeps before the restriction, on levels below 0 from x = 0.
 template <typename T>
-void batched_gs(pgmg_batch *b, int l, int sweeps, bool from_zero = false) {
+void batched_gs(pgmg_batch *b, int l, int sweeps, bool down, bool from_zero = false) {
 	if (sweeps <= 0) return;
+	for (int big = 0; big < 2; big++) {
+		const WorkList wl = wlist(b, list_index(l, L_TILE + big));
+		for (int s = 0; s < sweeps; s++)  // the last sweep writes x
+			launch_b_gs_tile<T>(b->stream, b->d_slots, wl, l, big != 0, b->tile_lds[l][big],
+					    s == 0 && down && (l > 0 || from_zero), ((sweeps - s) & 1) == 0);
+	}
 	for (int s = 0; s < sweeps; s++)
 		for (int q = 0; q < 4; q++) {
 			const bool fz = from_zero && s == 0;
@@ -340,7 +373,7 @@ template <typename T>
 void batched_cycle(pgmg_batch *b) {
 	const int L = b->max_nl;
 	for (int l = 0; l < L; l++) {
-		batched_gs<T>(b, l, b->opts.v_down + l, b->mixed && l == 0);
+		batched_gs<T>(b, l, b->opts.v_down + l, true, b->mixed && l == 0);
 		const WorkList wr = wlist(b, list_index(l, L_RES));
 		tuned(b, TC_RES, wr, [&](int c) { launch_b_residual<T>(b->stream, b->d_slots, wr, l, c); });
 		if (l == 0) {
@@ -357,7 +390,9 @@ void batched_cycle(pgmg_batch *b) {
 	for (int l = L - 1; l > 0; l--) {
 		const WorkList wi = wlist(b, list_index(l, L_INTERP));
 		tuned(b, TC_INTERP, wi, [&](int c) { launch_b_interp<T>(b->stream, b->d_slots, wi, l, c); });
-		batched_gs<T>(b, l - 1, b->opts.v_up + l - 1);
+		const WorkList wit = wlist(b, list_index(l, L_INTERP_T));
+		tuned(b, TC_INTERP, wit, [&](int c) { launch_b_interp<T>(b->stream, b->d_slots, wit, l, c, true); });
+		batched_gs<T>(b, l - 1, b->opts.v_up + l - 1, false);
 	}
 	if (b->mixed) {
 		// x += (double) x32 on level 0
@@ -445,6 +480,15 @@ int slot_setup(pgmg_batch *b, int s, const pgmg_dims *d, int family, uint64_t se
 			D.x32[l] = (float *)take(np * 4);
 			D.r32[l] = (float *)take(np * 4);
 		}
+	}
+	// Sweeps from x and back to x need an even number of them, sweeps from 0
+	// (level 0 of the mixed correction, and the levels below) any.
+	for (int l = 0; l < S.nl; l++) {
+		const int el = b->mixed ? 4 : 8;
+		S.tiles[l] = 0;
+		if (l == S.nl - 1 || batch_level_small(D.lv[l], el)) continue;
+		if (l > 0 || D.top_zero || (b->opts.v_down & 1) == 0)
+			S.tiles[l] = batch_tile(D.lv[l], el, D.tile[l], S.tile_big[l], S.tile_lds[l]);
 	}
 	const uint64_t np0 = (uint64_t)D.lv[0].npad;
 	if (b->mixed) D.res32 = (float *)take(np0 * 4); else D.res64 = (double *)take(np0 * 8);

@@ -182,6 +182,19 @@ __host__ __device__ inline int residual_blocks(const LevelView &L, int elem) {
 	return (waves + 3) / 4;
 }
 
+// What a launch of one-sweep tiles (launch_gs_tile) knows of its level, worked
+// out on the host.
+struct TileGeom {
+	int m, n, o, px, pxy, base;  // as LevelView, 32-bit
+	int pa, ablk;                // coefficient row and block pitch
+	int tj, tiles;               // tiles along j, and in all
+	int hx, nh;                  // x in LDS: row length, elements
+	int si, sj, sk;              // the thread count in LDS rows and planes: nt = si + hx*(sj + kTileHy*sk)
+	int np;                      // point pairs a row
+	int w1, w2, w3, w4;          // first wavefront of pairs 1, 2, 3; wavefronts in all
+	float inv_np, inv_hx;
+};
+
 // ---- batches of independent hierarchies (one per slot) ----
 const int kBatchMaxLevels = 16;
 // Device-side description of one slot's hierarchy.  Pointers of a precision
@@ -191,6 +204,7 @@ struct SlotDev {
 	int lu_active, lu_n;
 	int top_zero;  // mixed: the first level-0 sweep starts from x32 = 0 without reading it
 	LevelView lv[kBatchMaxLevels];
+	TileGeom tile[kBatchMaxLevels];  // of the levels that may take launch_b_gs_tile
 	double *A[kBatchMaxLevels], *x[kBatchMaxLevels], *r[kBatchMaxLevels];
 	float *A32[kBatchMaxLevels], *x32[kBatchMaxLevels], *r32[kBatchMaxLevels];
 	double *res64;     // residual scratch, top-level size
@@ -230,12 +244,24 @@ int batch_restrict_units(const LevelView &F, const LevelView &C);
 template <typename T> void launch_b_gs_pair(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int pair,
 					    bool from_zero = false, int chunk = 1, bool cross = false);
 template <typename T> void launch_b_gs_small(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int nsweeps);
+// One sweep of level `level` as launch_gs_tile's.  batch_tile fills the slot's
+// tile[level] and returns its tiles (work units), or 0 where the level does
+// not take these launches; big: it needs the larger of the two workgroup sizes
+// (a list holds slots of one size), lds: its LDS bytes (of a list, the most).
+// from_zero: x is 0 and not read; to_scratch: from x to the residual scratch,
+// else from there to x.
+int batch_tile(const LevelView &L, int elem, TileGeom &G, bool &big, size_t &lds);
+template <typename T> void launch_b_gs_tile(hipStream_t s, const SlotDev *slots, WorkList wl, int level, bool big,
+					    size_t lds, bool from_zero, bool to_scratch);
 template <typename T> void launch_b_residual(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk = 1,
 					     bool cross = false);
 void launch_b_residual_top(hipStream_t s, const SlotDev *slots, WorkList wl, bool to_f32, int chunk = 1, bool cross = false);
 void launch_b_reduce(hipStream_t s, const SlotDev *slots, WorkList wl, double *norms);
 template <typename T> void launch_b_restrict(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk = 1);
-template <typename T> void launch_b_interp(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk = 1);
+// to_scratch: the new x goes to the residual scratch (an odd number of
+// launch_b_gs_tile sweeps follows).
+template <typename T> void launch_b_interp(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk = 1,
+					   bool to_scratch = false);
 template <typename T> void launch_b_lu_solve(hipStream_t s, const SlotDev *slots, WorkList wl, int level);
 void launch_b_add_x(hipStream_t s, const SlotDev *slots, WorkList wl, int chunk = 1);
 

@@ -1109,16 +1109,6 @@ __device__ __forceinline__ void lds_pair_step(const typename Vec2<T>::type (&c)[
 	__syncthreads();
 }
 
-struct TileGeom {
-	int m, n, o, px, pxy, base;  // as LevelView, 32-bit
-	int pa, ablk;                // coefficient row and block pitch
-	int tj, tiles;               // tiles along j, and in all
-	int hx, nh;                  // x in LDS: row length, elements
-	int si, sj, sk;              // the thread count in LDS rows and planes: nt = si + hx*(sj + kTileHy*sk)
-	int np;                      // point pairs a row
-	int w1, w2, w3, w4;          // first wavefront of pairs 1, 2, 3; wavefronts in all
-	float inv_np, inv_hx;
-};
 constexpr int kTileHy = kTileJ + 7, kTileHz = kTileK + 3;  // rows and planes of x in LDS
 // Rows and planes of colour pair p in a tile.
 __host__ __device__ constexpr int tile_nj(int p) { return kTileJ / 2 + 3 - p; }
@@ -1130,12 +1120,9 @@ __device__ __forceinline__ int div_small(int a, float inv) { return (int)(((floa
 
 constexpr int kTileStage = 6;
 template <typename T, int NT>
-__global__ __launch_bounds__(NT) void k_gs_tile(TileGeom G, const T *__restrict__ A, const T *__restrict__ xin,
-						T *__restrict__ xout, const T *__restrict__ r) {
+__device__ __forceinline__ void gs_tile_body(const TileGeom &G, int tile, const T *__restrict__ A, const T *__restrict__ xin,
+					     T *__restrict__ xout, const T *__restrict__ r, T *__restrict__ xs) {
 	typedef typename Vec2<T>::type V2;
-	extern __shared__ __align__(16) char smem_[];
-	T *xs = (T *)smem_;
-	const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
 	const int tk = tile / G.tj;
 	const int J0 = (tile - tk * G.tj) * kTileJ, K0 = tk * kTileK;
 	const int hxy = G.hx * kTileHy;
@@ -1212,6 +1199,13 @@ __global__ __launch_bounds__(NT) void k_gs_tile(TileGeom G, const T *__restrict_
 	}
 }
 
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void k_gs_tile(TileGeom G, const T *__restrict__ A, const T *__restrict__ xin,
+						T *__restrict__ xout, const T *__restrict__ r) {
+	extern __shared__ __align__(16) char smem_[];
+	gs_tile_body<T, NT>(G, xcd_block((int)blockIdx.x, (int)gridDim.x), A, xin, xout, r, (T *)smem_);
+}
+
 // The launch of k_gs_tile on level L; false where the level does not take it:
 // periodic, more tiles than CUs (two or more to a CU run one after the other),
 // or rows too long for a tile to have a thread a point pair (16 wavefronts
@@ -1236,6 +1230,13 @@ bool tile_geom(const LevelView &L, TileGeom &G, int &nt, size_t &lds) {
 	G.si = nt % G.hx; G.sj = nt / G.hx % kTileHy; G.sk = nt / G.hx / kTileHy;
 	G.inv_np = 1.0f / (float)G.np; G.inv_hx = 1.0f / (float)G.hx;
 	return true;
+}
+
+int batch_tile(const LevelView &L, int elem, TileGeom &G, bool &big, size_t &lds) {
+	int nt = 0;
+	if (!(elem == 4 ? tile_geom<float>(L, G, nt, lds) : tile_geom<double>(L, G, nt, lds))) return 0;
+	big = nt > 512;
+	return G.tiles;
 }
 
 template <typename T>
@@ -3955,6 +3956,19 @@ __global__ __launch_bounds__(256) void kb_gs_pair(const SlotDev *__restrict__ sl
 // 768 threads: the most k_gs_pairs takes; a level with point pairs in more
 // wavefronts takes the one-point-a-thread form where it has a thread a point.
 constexpr int kBatchSmall = 768;
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void kb_gs_tile(const SlotDev *__restrict__ slots, WorkList wl, int level, int from_zero,
+						 int to_scratch) {
+	extern __shared__ __align__(16) char smem_[];
+	BATCH_LOOP
+		T *x = sx<T>(S, level), *other = sres<T>(S);
+		const TileGeom G = S->tile[level];
+		gs_tile_body<T, NT>(G, lu, sA<T>(S, level), from_zero ? nullptr : to_scratch ? x : other, to_scratch ? other : x,
+				    sr<T>(S, level), (T *)smem_);
+		__syncthreads();
+	}
+}
+
 template <typename T>
 __global__ __launch_bounds__(kBatchSmall) void kb_gs_small(const SlotDev *__restrict__ slots, WorkList wl, int level,
 							    int nsweeps) {
@@ -4041,11 +4055,12 @@ __global__ __launch_bounds__(256) void kb_restrict(const SlotDev *__restrict__ s
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void kb_interp(const SlotDev *__restrict__ slots, WorkList wl, int level) {
+__global__ __launch_bounds__(256) void kb_interp(const SlotDev *__restrict__ slots, WorkList wl, int level, int to_scratch) {
 	BATCH_LOOP
 		const LevelView F = S->lv[level - 1];
 		int ic, jc, kc;
-		if (cubes_unit(F, lu, ic, jc, kc)) interp_cube<T>(S->lv[level], F, sx<T>(S, level), sx<T>(S, level - 1), sx<T>(S, level - 1), ic, jc, kc);
+		T *xf = sx<T>(S, level - 1), *xo = to_scratch ? sres<T>(S) : xf;
+		if (cubes_unit(F, lu, ic, jc, kc)) interp_cube<T>(S->lv[level], F, sx<T>(S, level), xf, xo, ic, jc, kc);
 	}
 }
 
@@ -4103,6 +4118,18 @@ void launch_b_gs_small(hipStream_t s, const SlotDev *slots, WorkList wl, int lev
 	HIPCHECK_LAUNCH();
 }
 template <typename T>
+void launch_b_gs_tile(hipStream_t s, const SlotDev *slots, WorkList wl, int level, bool big, size_t lds, bool from_zero,
+		      bool to_scratch) {
+	if (wl.n <= 0) return;
+	constexpr int kMost = sizeof(T) == 4 ? 1024 : 768;
+	const dim3 grid(batch_grid(wl));
+	if (big)
+		hipLaunchKernelGGL((kb_gs_tile<T, kMost>), grid, dim3(kMost), lds, s, slots, wl, level, from_zero ? 1 : 0, to_scratch ? 1 : 0);
+	else
+		hipLaunchKernelGGL((kb_gs_tile<T, 512>), grid, dim3(512), lds, s, slots, wl, level, from_zero ? 1 : 0, to_scratch ? 1 : 0);
+	HIPCHECK_LAUNCH();
+}
+template <typename T>
 void launch_b_residual(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk, bool cross) {
 	if (wl.n <= 0) return;
 	const dim3 grid(batch_grid(wl, chunk)), block(64, 4);
@@ -4129,9 +4156,9 @@ void launch_b_restrict(hipStream_t s, const SlotDev *slots, WorkList wl, int lev
 	HIPCHECK_LAUNCH();
 }
 template <typename T>
-void launch_b_interp(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk) {
+void launch_b_interp(hipStream_t s, const SlotDev *slots, WorkList wl, int level, int chunk, bool to_scratch) {
 	if (wl.n <= 0) return;
-	hipLaunchKernelGGL(kb_interp<T>, dim3(batch_grid(wl, chunk)), dim3(64, 4), 0, s, slots, wl, level);
+	hipLaunchKernelGGL(kb_interp<T>, dim3(batch_grid(wl, chunk)), dim3(64, 4), 0, s, slots, wl, level, to_scratch ? 1 : 0);
 	HIPCHECK_LAUNCH();
 }
 template <typename T>
@@ -4170,7 +4197,8 @@ void launch_b_add_x(hipStream_t s, const SlotDev *slots, WorkList wl, int chunk)
 	template void launch_b_gs_small<T>(hipStream_t, const SlotDev *, WorkList, int, int); \
 	template void launch_b_residual<T>(hipStream_t, const SlotDev *, WorkList, int, int, bool); \
 	template void launch_b_restrict<T>(hipStream_t, const SlotDev *, WorkList, int, int); \
-	template void launch_b_interp<T>(hipStream_t, const SlotDev *, WorkList, int, int); \
+	template void launch_b_interp<T>(hipStream_t, const SlotDev *, WorkList, int, int, bool); \
+	template void launch_b_gs_tile<T>(hipStream_t, const SlotDev *, WorkList, int, bool, size_t, bool, bool); \
 	template void launch_b_lu_solve<T>(hipStream_t, const SlotDev *, WorkList, int);
 INST(double)
 INST(float)

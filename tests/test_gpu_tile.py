@@ -61,3 +61,24 @@ def test_cycles_bitwise(precision, v_down, v_up):
         c, _ = h.solve(1e-7, 40)
         assert c == cycles
         assert np.array_equal(h.get_x(), mg.get_x(0))
+
+
+@pytest.mark.parametrize("precision", [P.PREC_FP64, P.PREC_MIXED])
+@pytest.mark.parametrize("v_down,v_up", [(2, 2), (1, 2), (3, 1), (0, 1)])
+def test_batch_equals_alone(precision, v_down, v_up):
+    # levels with and without tiles, of both workgroup sizes, at levels 0 to 2;
+    # the second batch has too many tiles at a level for tile launches
+    dims = [(34, 40, 27), (20, 13, 11), (65, 70, 40), (17, 17, 17), (79, 20, 18), (50, 49, 33)]
+    for repeat in (1, 8):
+        with P.Batch(1 << 31, max_slots=64, precision=precision, v_down=v_down, v_up=v_up) as batch:
+            slots = [(d, batch.admit(*d, P.FAM_Q1_ANISO, 70 + q, 1e-6, 12)) for _ in range(repeat)
+                     for q, d in enumerate(dims)]
+            batch.run()
+            for q, (d, s) in enumerate(slots):
+                print("case", d, repeat, flush=True)
+                with P.Hierarchy(*d, precision=precision, v_down=v_down, v_up=v_up) as h:
+                    h.generate_problem(P.FAM_Q1_ANISO, 70 + q % len(dims))
+                    h.compute_rats()
+                    c, _ = h.solve(1e-6, 12, check=False)
+                    assert batch.status(s)[1] == c
+                    assert np.array_equal(batch.get_x(s), h.get_x())
