@@ -3548,39 +3548,241 @@ void launch_lu_factor(hipStream_t s, int N, double *LU, int *ipiv, int *info) {
 }
 
 // dgetrs('N') on one workgroup (region_tr.cc:544-555): interchanges, then
-// column-oriented forward and back substitution in FP64, one barrier per
-// column.  r and x are in the level layout and type T.
+// column-oriented forward and back substitution in FP64.  r and x are in the
+// level layout and type T.
+//
+// Bound by the serial chain over the N unknowns and, behind it, by one CU
+// reading the factor.  Row block R (64 rows, one a lane) belongs to wavefront
+// R mod 8, which applies the columns to it 32 at a time: a column's unknown
+// is read out of a lane (v_readlane), the block's own columns form the chain,
+// and the coefficients of its next two pieces of work are in flight
+// meanwhile (one piece ahead: 138 us below).  One barrier per 32 columns.  Every row subtracts its terms one by one in column order,
+// as the column-by-column loop, so x is the same.
+//
+// Without interchanges the factor keeps the operator's band (half width bw =
+// 1 + m + mn in the order of the points): blocks outside it, which are zero,
+// are not read.  With interchanges U's upper half width is at most 2 bw and L
+// is taken as full; so are both with periodic axes.
+//
+// 11x7x9 unknowns: 675 us a solve with a barrier a column, 107 us so (122 with
+// four wavefronts of twice the registers).
+const int kLuWaves = 8;
+const int kLuMax = 2048;  // enable_exact takes fewer points than this
+
+// The half width of the band of L's bottom operator, and N where it has none.
+__device__ __forceinline__ int lu_band(const LevelView &L, int N) {
+	return L.prd ? N : min(N, 1 + L.m + L.m * L.n);
+}
+
+// Correctly rounded n / d from y = 1/d rounded to nearest: the second
+// correction starts from a faithful quotient and its remainder is exact
+// (Markstein).  Valid where no step leaves the normal range: see lu_div_ok.
+__device__ __forceinline__ double lu_div(double n, double d, double y) {
+	double q = n * y;
+	q = fma(fma(-d, q, n), y, q);
+	return fma(fma(-d, q, n), y, q);
+}
+// |n| in [2^-500, 2^500], or 0 (|d| in [2^-200, 2^200] is checked by itself).
+__device__ __forceinline__ bool lu_div_ok(double n) {
+	const unsigned e = (unsigned)(__double_as_longlong(n) >> 52) & 0x7ff;
+	return (e >= 1023 - 500 && e < 1023 + 500) || n == 0.0;
+}
+
+// A wavefront's pieces of work in the order it takes them: row block R,
+// columns 32 cb .. 32 cb + 31; forward cb ascends and, within it, R, from the
+// diagonal block's; back both descend.  reach: the half width of the band.
+template <bool FORWARD>
+struct LuWalk {
+	int cb, R, w, ncb, reach;
+	__device__ __forceinline__ LuWalk(int w_, int nblk, int reach_) : w(w_), ncb(2 * nblk), reach(reach_) {
+		cb = FORWARD ? 0 : ncb - 1;
+		first();
+		settle();
+	}
+	__device__ __forceinline__ void first() {
+		const int D = cb >> 1;
+		R = FORWARD ? D + ((w - D) & (kLuWaves - 1)) : D - ((D - w) & (kLuWaves - 1));
+	}
+	__device__ __forceinline__ bool done() const { return FORWARD ? cb >= ncb : cb < 0; }
+	// to the next piece at or after (cb, R)
+	__device__ __forceinline__ void settle() {
+		while (!done() && (FORWARD ? R > min(ncb / 2 - 1, (32 * cb + 31 + reach) / 64) : R < max(0, 32 * cb - reach) / 64)) {
+			cb += FORWARD ? 1 : -1;
+			first();
+		}
+	}
+	__device__ __forceinline__ void next() {
+		R += FORWARD ? kLuWaves : -kLuWaves;
+		settle();
+	}
+};
+
+// A piece's coefficients in flight.
+struct LuPiece {
+	int cb, R;      // cb outside the factor: none
+	double d;       // back, diagonal block: the row's diagonal entry
+	double a[32];
+	template <bool FORWARD>
+	__device__ __forceinline__ void load(LuWalk<FORWARD> &walk, int N, const double *__restrict__ LU) {
+		cb = walk.cb;
+		R = walk.R;
+		if (walk.done()) return;
+		// rows and columns past the end repeat the last ones (their terms
+		// are not used, or are multiplied by 0)
+		const int row = min(64 * R + (int)threadIdx.x % 64, N - 1);
+#pragma unroll
+		for (int c = 0; c < 32; c++) a[c] = LU[(long long)min(32 * cb + c, N - 1) * N + row];
+		if (!FORWARD) d = LU[(long long)row * N + row];
+		walk.next();
+	}
+};
+
+// Forward substitution of a piece.
+__device__ __forceinline__ void lu_forward(const LuPiece &p, double *__restrict__ xs) {
+	const int lane = threadIdx.x % 64;
+	double xr = xs[64 * p.R + lane];
+	if (p.R != p.cb / 2) {
+		const double xc = xs[32 * p.cb + (lane & 31)];
+#pragma unroll
+		for (int c = 0; c < 32; c++) {
+			const double t = read_lane(xc, c) * p.a[c];
+			xr -= t;
+		}
+		xs[64 * p.R + lane] = xr;
+		return;
+	}
+	const int h = p.cb & 1;
+	int l = lane - 32 * h;
+	asm volatile("" : "+v"(l));  // keeps 32 loop-invariant masks out of the registers
+#pragma unroll
+	for (int c = 0; c < 32; c++) {
+		const double t = read_lane(xr, 32 * h + c) * (l > c ? p.a[c] : 0.0);
+		xr -= t;
+	}
+	// other wavefronts may be reading the block's first half
+	if (l >= 0) xs[64 * p.R + lane] = xr;
+}
+
+// Back substitution of a piece.
+__device__ __forceinline__ void lu_back(const LuPiece &p, double *__restrict__ xs, int N, const double *__restrict__ LU) {
+	const int lane = threadIdx.x % 64, row = 64 * p.R + lane;
+	const double x0 = xs[row];
+	double xr = x0;
+	if (p.R != p.cb / 2) {
+		const double xc = xs[32 * p.cb + (lane & 31)];
+#pragma unroll
+		for (int c = 31; c >= 0; c--) {
+			const double t = read_lane(xc, c) * p.a[c];
+			xr -= t;
+		}
+		xs[row] = xr;
+		return;
+	}
+	const int h = p.cb & 1;
+	int l = lane - 32 * h;
+	asm volatile("" : "+v"(l));
+	const double d = row < N ? p.d : 1.0, y = 1.0 / d;
+	const unsigned ed = (unsigned)(__double_as_longlong(d) >> 52) & 0x7ff;
+	bool bad = ed < 1023 - 200 || ed >= 1023 + 200;
+	double sol = 0.0;
+#pragma unroll
+	for (int c = 31; c >= 0; c--) {
+		const double q = lu_div(xr, d, y);
+		if (l == c) {
+			sol = q;
+			bad |= !lu_div_ok(xr);
+		}
+		const double t = read_lane(q, 32 * h + c) * (l < c ? p.a[c] : 0.0);
+		xr -= t;
+	}
+	if (__ballot(bad)) {  // again, with the division
+		xr = x0;
+		for (int c = 31; c >= 0; c--) {
+			const double q = xr / d;
+			if (l == c) sol = q;
+			const int col = 32 * p.cb + c;
+			const double t = read_lane(q, 32 * h + c) * (l < c && col < N ? LU[(long long)col * N + min(row, N - 1)] : 0.0);
+			xr -= t;
+		}
+	}
+	if (l < 32) xs[row] = l < 0 ? xr : sol;
+}
+
 template <typename T>
 __device__ __forceinline__ void lu_solve_body(const LevelView &L, int N, const double *__restrict__ LU,
 					      const int *__restrict__ ipiv, const T *__restrict__ r, T *__restrict__ x) {
-	__shared__ double xs[1024];
+	__shared__ double xs[kLuMax];
+	__shared__ int sp[kLuMax];
 	const int tid = threadIdx.x, nt = blockDim.x;
-	for (int q = tid; q < N; q += nt) {
-		const int i = q % L.m, j = (q / L.m) % L.n, k = q / (L.m * L.n);
-		xs[q] = (double)r[idx3(L, i, j, k)];
-	}
-	__syncthreads();
-	if (tid == 0) {
-		for (int c = 0; c < N; c++) {
-			const int p = ipiv[c];
-			if (p != c) { const double t = xs[c]; xs[c] = xs[p]; xs[p] = t; }
+	const int w = __builtin_amdgcn_readfirstlane(tid / 64);
+	const int nblk = (N + 63) / 64, ncb = 2 * nblk;
+	int moved = 0;
+	for (int q = tid; q < 64 * nblk; q += nt) {
+		double v = 0.0;
+		if (q < N) {
+			const int i = q % L.m, j = (q / L.m) % L.n, k = q / (L.m * L.n);
+			v = (double)r[idx3(L, i, j, k)];
+			sp[q] = ipiv[q];
+			moved |= sp[q] != q;
 		}
+		xs[q] = v;
+	}
+	moved = __syncthreads_or(moved);
+	if (moved) {
+		if (tid == 0)
+			for (int c = 0; c < N; c++) {
+				const int p = sp[c];
+				if (p != c) { const double t = xs[c]; xs[c] = xs[p]; xs[p] = t; }
+			}
+		__syncthreads();
+	}
+	const int band = lu_band(L, N);
+	const int bl = moved ? N : band, bu = moved ? min(N, 2 * band) : band;
+	LuPiece p0, p1, p2;
+
+	// A piece below (above) the diagonal needs its columns' unknowns, final
+	// and written, which the diagonal piece's wavefront does before it comes
+	// to barrier number cb + 1 (ncb - cb).
+	{
+		LuWalk<true> walk(w, nblk, bl);
+		int passed = 0;
+		p0.load(walk, N, LU);
+		p1.load(walk, N, LU);
+		p2.load(walk, N, LU);
+		const auto step = [&](LuPiece &p) {
+			if (p.cb >= ncb) return false;
+			for (const int need = p.R != p.cb / 2 ? p.cb + 1 : p.cb; passed < need; passed++) __syncthreads();
+			lu_forward(p, xs);
+			p.load(walk, N, LU);
+			return true;
+		};
+		while (step(p0) && step(p1) && step(p2)) {
+		}
+		for (; passed < ncb; passed++) __syncthreads();
 	}
 	__syncthreads();
-	for (int c = 0; c < N; c++) {
-		const double v = xs[c];
-		if (v != 0.0)
-			for (int rr = c + 1 + tid; rr < N; rr += nt) xs[rr] -= v * LU[rr + (long long)c * N];
-		__syncthreads();
+	// rows past the end solve to 0
+	if (tid < 64 && 64 * nblk - 64 + tid >= N) xs[64 * nblk - 64 + tid] = 0.0;
+	__syncthreads();
+	{
+		LuWalk<false> walk(w, nblk, bu);
+		int passed = 0;
+		p0.load(walk, N, LU);
+		p1.load(walk, N, LU);
+		p2.load(walk, N, LU);
+		const auto step = [&](LuPiece &p) {
+			if (p.cb < 0) return false;
+			const int done = ncb - 1 - p.cb;
+			for (const int need = p.R != p.cb / 2 ? done + 1 : done; passed < need; passed++) __syncthreads();
+			lu_back(p, xs, N, LU);
+			p.load(walk, N, LU);
+			return true;
+		};
+		while (step(p0) && step(p1) && step(p2)) {
+		}
+		for (; passed < ncb; passed++) __syncthreads();
 	}
-	for (int c = N - 1; c >= 0; c--) {
-		const double v = xs[c] / LU[c + (long long)c * N];
-		__syncthreads();
-		if (tid == 0) xs[c] = v;
-		if (v != 0.0)
-			for (int rr = tid; rr < c; rr += nt) xs[rr] -= v * LU[rr + (long long)c * N];
-		__syncthreads();
-	}
+	__syncthreads();
 	for (int q = tid; q < N; q += nt) {
 		const int i = q % L.m, j = (q / L.m) % L.n, k = q / (L.m * L.n);
 		x[idx3(L, i, j, k)] = (T)xs[q];
@@ -3588,14 +3790,14 @@ __device__ __forceinline__ void lu_solve_body(const LevelView &L, int N, const d
 }
 
 template <typename T>
-__global__ __launch_bounds__(1024) void k_lu_solve(LevelView L, int N, const double *__restrict__ LU,
+__global__ __launch_bounds__(64 * kLuWaves) void k_lu_solve(LevelView L, int N, const double *__restrict__ LU,
 						   const int *__restrict__ ipiv, const T *__restrict__ r, T *__restrict__ x) {
 	lu_solve_body<T>(L, N, LU, ipiv, r, x);
 }
 
 template <typename T>
 void launch_lu_solve(hipStream_t s, const LevelView &L, int N, const double *LU, const int *ipiv, const T *r, T *x) {
-	hipLaunchKernelGGL(k_lu_solve<T>, dim3(1), dim3(1024), 0, s, L, N, LU, ipiv, r, x);
+	hipLaunchKernelGGL(k_lu_solve<T>, dim3(1), dim3(64 * kLuWaves), 0, s, L, N, LU, ipiv, r, x);
 	HIPCHECK_LAUNCH();
 }
 
@@ -4065,7 +4267,7 @@ __global__ __launch_bounds__(256) void kb_interp(const SlotDev *__restrict__ slo
 }
 
 template <typename T>
-__global__ __launch_bounds__(1024) void kb_lu_solve(const SlotDev *__restrict__ slots, WorkList wl, int level) {
+__global__ __launch_bounds__(64 * kLuWaves) void kb_lu_solve(const SlotDev *__restrict__ slots, WorkList wl, int level) {
 	BATCH_LOOP
 		(void)lu;
 		lu_solve_body<T>(S->lv[level], S->lu_n, slot_ptr(S->LU), slot_ptr(S->ipiv), sr<T>(S, level), sx<T>(S, level));
@@ -4164,7 +4366,7 @@ void launch_b_interp(hipStream_t s, const SlotDev *slots, WorkList wl, int level
 template <typename T>
 void launch_b_lu_solve(hipStream_t s, const SlotDev *slots, WorkList wl, int level) {
 	if (wl.n <= 0) return;
-	hipLaunchKernelGGL(kb_lu_solve<T>, dim3(batch_grid(wl)), dim3(1024), 0, s, slots, wl, level);
+	hipLaunchKernelGGL(kb_lu_solve<T>, dim3(batch_grid(wl)), dim3(64 * kLuWaves), 0, s, slots, wl, level);
 	HIPCHECK_LAUNCH();
 }
 void launch_b_add_x(hipStream_t s, const SlotDev *slots, WorkList wl, int chunk) {
