@@ -179,6 +179,7 @@ struct pgmg_batch {
 	hipGraphExec_t cycle_graph = nullptr;
 	int plan_steps = 0;   // consecutive steps on the current plan
 	long long graph_launches = 0;
+	HostReadout readout;
 };
 
 namespace {
@@ -742,13 +743,7 @@ int pgmg_batch_get_x(pgmg_batch *b, int slot, double *x) {
 	// a slot still in set-up waits for its own set-up only, not for later admissions
 	if (S.state == ST_SETUP) BHIP(hipEventSynchronize(S.ready));
 	const LevelView &L = S.dev.lv[0];
-	const long long N = (long long)L.m * L.n * L.o;
-	double *stage = nullptr;
-	BHIP(hipMallocAsync((void **)&stage, sizeof(double) * (size_t)N, b->stream));
-	launch_unpack_vec(b->stream, L, S.dev.x[0], stage, 0, N);
-	BHIP(hipMemcpyAsync(x, stage, sizeof(double) * N, hipMemcpyDeviceToHost, b->stream));
-	BHIP(hipFreeAsync(stage, b->stream));
-	BHIP(hipStreamSynchronize(b->stream));
+	BHIP(b->readout.copy(b->stream, L, S.dev.x[0], x));
 	return PGMG_OK;
 }
 

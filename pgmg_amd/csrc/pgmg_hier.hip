@@ -103,6 +103,7 @@ struct pgmg_hier {
 	long long prof_launches = 0, prof_points = 0;
 	double prof_ms = 0;
 	bool capturing = false;
+	HostReadout readout;
 };
 
 namespace {
@@ -871,16 +872,15 @@ int pgmg_lu_active(const pgmg_hier *h, int *active) {
 static int vec_io(pgmg_hier *h, int level, double *dptr, const double *hin, double *hout) {
 	Level &L = h->lev[level];
 	const long long N = L.points();
+	if (!hin) {
+		const hipError_t e = h->readout.copy(h->stream, L.v, dptr, hout);
+		if (e != hipSuccess) return fail(PGMG_ERR_HIP, "vector transfer: %s", hipGetErrorString(e));
+		return PGMG_OK;
+	}
 	double *stage = nullptr;
 	HIP_TRY(hipMalloc(&stage, sizeof(double) * (size_t)N));
-	hipError_t e = hipSuccess;
-	if (hin) {
-		e = hipMemcpyAsync(stage, hin, sizeof(double) * N, hipMemcpyHostToDevice, h->stream);
-		if (e == hipSuccess) launch_pack_vec(h->stream, L.v, stage, dptr, 0, N);
-	} else {
-		launch_unpack_vec(h->stream, L.v, dptr, stage, 0, N);
-		e = hipMemcpyAsync(hout, stage, sizeof(double) * N, hipMemcpyDeviceToHost, h->stream);
-	}
+	hipError_t e = hipMemcpyAsync(stage, hin, sizeof(double) * N, hipMemcpyHostToDevice, h->stream);
+	if (e == hipSuccess) launch_pack_vec(h->stream, L.v, stage, dptr, 0, N);
 	if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
 	hipFree(stage);
 	if (e != hipSuccess) return fail(PGMG_ERR_HIP, "vector transfer: %s", hipGetErrorString(e));

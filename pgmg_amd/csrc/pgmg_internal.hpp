@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <cstddef>
+#include <mutex>
 
 namespace pgmg {
 
@@ -381,6 +382,22 @@ void launch_unpack_vec(hipStream_t s, const LevelView &L, const double *padded, 
 void launch_pack_op(hipStream_t s, const LevelView &L, const double *compact27, double *A, long long p0, long long count,
 		    int *dense = nullptr);
 void launch_unpack_op(hipStream_t s, const LevelView &L, const double *A, double *compact27, long long p0, long long count);
+// Level vectors to host arrays, point-major, through a pinned buffer kept for
+// the next call (at most kSlots chunks: pgmg_readout.hip).  Calls of several
+// threads take turns.
+class HostReadout {
+public:
+	~HostReadout();
+	// The grid points of d to out; out is complete on return.
+	hipError_t copy(hipStream_t s, const LevelView &L, const double *d, double *out);
+	static const int kSlots = 16;
+
+private:
+	std::mutex mu;
+	double *buf = nullptr;
+	size_t cap = 0;
+	hipEvent_t ev[kSlots] = {};
+};
 // Elementwise helpers.
 template <typename T> void launch_fill(hipStream_t s, T *p, long long n, T v);
 void launch_round_f32(hipStream_t s, const double *src, float *dst, long long n);
