@@ -265,6 +265,21 @@ bool gs_use_tile(const pgmg_hier *h, int level, int mode) {
 // only with gs_use_tile, X_ZERO with gs_from_zero_ok or gs_use_tile.
 enum XStart { X_LEVEL, X_SCRATCH, X_ZERO };
 
+// One forward colour sweep in place on the per-row kernels.
+template <typename T>
+void colour_sweep(pgmg_hier *h, Level &L) {
+	launch_halo_wrap<T>(h->stream, L.v, lx<T>(L));
+	// The colour-pair row kernels read the halo point m from memory where a
+	// row ends, except in the point out of a row of ppl*q+1 points, which
+	// takes it as zero: with a periodic x axis such rows use the per-class
+	// kernel.
+	if ((L.v.prd & 1) && row_lanes(L.v.m, (int)sizeof(T)).ext) {
+		for (int c = 0; c < 8; c++) launch_gs_colour<T>(h->stream, L.v, lA<T>(L), lx<T>(L), lr<T>(L), c);
+	} else {
+		for (int q = 0; q < 4; q++) launch_gs_pair<T>(h->stream, L.v, lA<T>(L), lx<T>(L), lr<T>(L), q, false);
+	}
+}
+
 template <typename T>
 void tile_sweeps(pgmg_hier *h, int level, int nsweeps, XStart from) {
 	Level &L = h->lev[level];
@@ -274,7 +289,7 @@ void tile_sweeps(pgmg_hier *h, int level, int nsweeps, XStart from) {
 		// an odd number of exchanges would leave x in the scratch: one
 		// sweep in place
 		ProfScope ps(h, KC_GS, level, L.points());
-		for (int q = 0; q < 4; q++) launch_gs_pair<T>(h->stream, L.v, lA<T>(L), x, lr<T>(L), q, false);
+		colour_sweep<T>(h, L);
 		left--;
 	}
 	const T *in = from == X_ZERO ? nullptr : from == X_SCRATCH ? other : x;
@@ -294,17 +309,16 @@ void op_gs(pgmg_hier *h, int level, int mode, int nsweeps, XStart from = X_LEVEL
 	h->gs_count += nsweeps;
 	if (nsweeps <= 0) return;
 	const bool use_small = gs_use_small<T>(h, L, mode);
+	if (gs_use_tile<T>(h, level, mode)) {
+		tile_sweeps<T>(h, level, nsweeps, from);
+		return;
+	}
 	if (L.v.prd && !use_small) {
 		// Periodic axes: the ghost copies are refreshed before each pass
 		// (region.cc:361, 457), then the pass runs on the per-point kernels,
 		// which read the halo like any neighbour.  (The one-workgroup kernel
 		// refreshes them itself.)
 		const int tmax = (L.v.m - 1) + 2 * (L.v.n - 1) + 4 * (L.v.o - 1);
-		// The colour-pair row kernels read the halo point m from memory where
-		// a row ends, except in the point out of a row of ppl*q+1 points,
-		// which takes it as zero: with a periodic x axis such rows use the
-		// per-class kernel.
-		const bool pair_ok = !(L.v.prd & 1) || !row_lanes(L.v.m, (int)sizeof(T)).ext;
 		if (exact && !mode && sA<T>(L) && h->ops_ready) {
 			// plane-skewed copies, ghosts refreshed on them before each sweep
 			launch_skew_vec<T>(h->stream, L.v, L.sv, lx<T>(L), sx<T>(L), true);
@@ -320,16 +334,17 @@ void op_gs(pgmg_hier *h, int level, int mode, int nsweeps, XStart from = X_LEVEL
 		for (int s = 0; s < nsweeps; s++)
 			for (int pass = 0; pass < (mode ? 2 : 1); pass++) {
 				ProfScope ps(h, KC_GS, level, L.points());
+				if (!exact && pass == 0) {
+					colour_sweep<T>(h, L);
+					continue;
+				}
 				launch_halo_wrap<T>(h->stream, L.v, lx<T>(L));
 				if (exact) {
 					for (int tt = 0; tt <= tmax; tt++)
 						launch_gs_plane<T>(h->stream, L.v, lA<T>(L), lx<T>(L), lr<T>(L), pass ? tmax - tt : tt);
-				} else if (pass == 0 && pair_ok) {
-					for (int q = 0; q < 4; q++)
-						launch_gs_pair<T>(h->stream, L.v, lA<T>(L), lx<T>(L), lr<T>(L), q, false);
 				} else {
-					for (int c = 0; c < 8; c++)
-						launch_gs_colour<T>(h->stream, L.v, lA<T>(L), lx<T>(L), lr<T>(L), pass ? 7 - c : c);
+					for (int c = 7; c >= 0; c--)
+						launch_gs_colour<T>(h->stream, L.v, lA<T>(L), lx<T>(L), lr<T>(L), c);
 				}
 			}
 		return;
@@ -337,10 +352,6 @@ void op_gs(pgmg_hier *h, int level, int mode, int nsweeps, XStart from = X_LEVEL
 	if (use_small) {
 		ProfScope ps(h, KC_GS, level, L.points() * nsweeps * (mode ? 2 : 1));
 		launch_gs_small<T>(h->stream, L.v, lA<T>(L), lx<T>(L), lr<T>(L), nsweeps, mode, exact ? 1 : 0);
-		return;
-	}
-	if (gs_use_tile<T>(h, level, mode)) {
-		tile_sweeps<T>(h, level, nsweeps, from);
 		return;
 	}
 	const int tmax = (L.v.m - 1) + 2 * (L.v.n - 1) + 4 * (L.v.o - 1);

@@ -187,6 +187,7 @@ __host__ __device__ inline int residual_blocks(const LevelView &L, int elem) {
 // out on the host.
 struct TileGeom {
 	int m, n, o, px, pxy, base;  // as LevelView, 32-bit
+	int prd;                     // as LevelView
 	int pa, ablk;                // coefficient row and block pitch
 	int tj, tiles;               // tiles along j, and in all
 	int hx, nh;                  // x in LDS: row length, elements

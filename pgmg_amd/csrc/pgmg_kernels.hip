@@ -1037,12 +1037,16 @@ void launch_gs_pair(hipStream_t s, const LevelView &L, const T *A, T *x, const T
 // arithmetic and order as in gs_point.  Indices are 32-bit with 24-bit
 // products, and the host passes what it can work out (TileGeom).
 // Only grid points of xin and xout are accessed (their halos may hold
-// anything), and positions outside the grid count as 0 (loaded from r's
-// first, halo, element), so the level must not be periodic.
+// anything).  Positions outside the grid count as 0 (loaded from r's first
+// element, before the halo); next to the grid on a periodic axis they are the
+// wrapped points' x on entry, which no update of the sweep changes, as the
+// ghost copies refreshed before a sweep.
 //
 // Measured, launches back to back: 17^3 6.5 us a sweep against 14.5 (FP32;
 // FP64 6.7 against 14.9), 33^3 6.8 against 14.5 (FP64 7.2 against 14.7); 65^3,
 // whose 561 tiles are more than two to a CU, 24 against 16 (not used there).
+// Periodic FP64 (the other way takes five launches, the ghosts' refresh among
+// them): 24x20x28 6.0 us a sweep against 22, 48x40x56, 280 tiles, 14.5 against 22.
 constexpr int kTileJ = 4, kTileK = 2;
 // One colour pair of a level (or tile) with x in LDS: the threads that are on
 // update their point pair (i0, i0+1), xl its even point in LDS, from the pair's
@@ -1134,9 +1138,14 @@ __device__ __forceinline__ void gs_tile_body(const TileGeom &G, int tile, const 
 	int si = tid - __mul24(row0, G.hx), sk = row0 / kTileHy, sj = row0 - sk * kTileHy;
 	auto stage = [&]() -> T {
 		// LDS position (si, sj, sk) is grid point (si-1, jb+sj, kb+sk)
-		const int j = jb + sj, k = kb + sk;
-		const bool in = xin && (unsigned)(si - 1) < (unsigned)G.m && (unsigned)j < (unsigned)G.n && (unsigned)k < (unsigned)G.o;
-		const int off = in ? G.base + si - 1 + __mul24(j, G.px) + __mul24(k, G.pxy) : 0;
+		int i = si - 1, j = jb + sj, k = kb + sk;
+		if (G.prd) {  // the ghosts next to the grid are the wrapped points
+			if (G.prd & 1) i = i == -1 ? G.m - 1 : i == G.m ? 0 : i;
+			if (G.prd & 2) j = j == -1 ? G.n - 1 : j == G.n ? 0 : j;
+			if (G.prd & 4) k = k == -1 ? G.o - 1 : k == G.o ? 0 : k;
+		}
+		const bool in = xin && (unsigned)i < (unsigned)G.m && (unsigned)j < (unsigned)G.n && (unsigned)k < (unsigned)G.o;
+		const int off = in ? G.base + i + __mul24(j, G.px) + __mul24(k, G.pxy) : 0;
 		const T v = (in ? xin : r)[off];
 		si += G.si; sj += G.sj; sk += G.sk;
 		if (si >= G.hx) { si -= G.hx; sj++; }
@@ -1207,25 +1216,25 @@ __global__ __launch_bounds__(NT) void k_gs_tile(TileGeom G, const T *__restrict_
 }
 
 // The launch of k_gs_tile on level L; false where the level does not take it:
-// periodic, more tiles than CUs (two or more to a CU run one after the other),
-// or rows too long for a tile to have a thread a point pair (16 wavefronts
+// more tiles than CUs (two or more to a CU run one after the other; two pay
+// where the other way refreshes ghosts and reads all 27 planes), or rows too long for a tile to have a thread a point pair (16 wavefronts
 // of 128 registers in FP32, 12 of 168 in FP64) or for its x to fit LDS.
 template <typename T>
 bool tile_geom(const LevelView &L, TileGeom &G, int &nt, size_t &lds) {
-	if (L.prd) return false;
 	G.np = (L.m + 1) / 2;
 	int w[5] = {0, 0, 0, 0, 0};
 	for (int p = 0; p < 4; p++) w[p + 1] = w[p] + (tile_nj(p) * tile_nk(p) * G.np + 63) / 64;
 	G.hx = (L.m + 3) & ~1;  // i = -1 .. m+1, even: the pairs (i0-1, i0) and (i0+1, i0+2) are aligned
 	G.tj = (L.n + kTileJ - 1) / kTileJ;
 	const long long tiles = (long long)G.tj * ((L.o + kTileK - 1) / kTileK), nh = (long long)G.hx * kTileHy * kTileHz;
-	if (w[4] > (sizeof(T) == 4 ? 16 : 12) || nh * (long long)sizeof(T) > kSmallLdsBytes || tiles > 256) return false;
+	if (w[4] > (sizeof(T) == 4 ? 16 : 12) || nh * (long long)sizeof(T) > kSmallLdsBytes || tiles > (L.prd && !L.cross ? 512 : 256))
+		return false;
 	nt = w[4] <= 8 ? 512 : sizeof(T) == 4 ? 1024 : 768;
 	lds = sizeof(T) * (size_t)nh;
 	G.tiles = (int)tiles;
 	G.nh = (int)nh;
 	G.w1 = w[1]; G.w2 = w[2]; G.w3 = w[3]; G.w4 = w[4];
-	G.m = L.m; G.n = L.n; G.o = L.o; G.px = L.px; G.pxy = (int)L.pxy; G.base = (int)L.base;
+	G.m = L.m; G.n = L.n; G.o = L.o; G.px = L.px; G.pxy = (int)L.pxy; G.base = (int)L.base; G.prd = L.prd;
 	G.pa = L.pa; G.ablk = (int)ablock(L);
 	G.si = nt % G.hx; G.sj = nt / G.hx % kTileHy; G.sk = nt / G.hx / kTileHy;
 	G.inv_np = 1.0f / (float)G.np; G.inv_hx = 1.0f / (float)G.hx;
