@@ -247,9 +247,13 @@ __device__ __forceinline__ bool zero_row(int cj, int ck, int dj, int dk) {
 // after the next segment's loads (one counter tracks loads and stores in
 // issue order, so a load issued after a store would wait for it); the only
 // loads they overtake are the next segment's lane-0 reads of s0-1 and s0,
-// which feed the even point that lane takes from the hand-over.  Per-point
-// arithmetic and the colour order are those of k_gs_colour, so the result is
-// bit-identical.  j and k must be wavefront-uniform.
+// which feed the even point that lane takes from the hand-over.  A lane
+// stores its points as one vector (the handed-over point with lane 0's, so
+// lane 63 stores a point out only at the row's end): stored one by one, each
+// write-through moved its own part of a line, and a 257^3 FP64 launch wrote
+// 67 MB for its 34 (99.3 us a launch, 95.7 so; 385x257x321 FP32 197 and 189).
+// Per-point arithmetic and the colour order are those of k_gs_colour, so the
+// result is bit-identical.  j and k must be wavefront-uniform.
 //
 // The point out's 27 coefficients and the x of the point after it in each of
 // its 9 rows are loaded by lanes 0..26 and 0..8, one load each, and lane 63
@@ -371,8 +375,8 @@ __device__ __forceinline__ void gs_pair_row(const LevelView &L, const T *__restr
 				}
 			}
 		}
-		if (pE) st_row<T>(xr, pob, pe);
-		if (pO) st_row<T>(xr + 1, pob, po);
+		if (pO) { V2 v; v.x = pe; v.y = po; st_row<V2>(xr, pob, v); }
+		else if (pE) st_row<T>(xr, pob, pe);
 		if (pZ) st_row<T>(xr, pob + 2u * (uint32_t)sizeof(T), pz);
 		// even points: every neighbour still holds its old value
 		T xe = (T)0, xz = (T)0, xo = (T)0;
@@ -394,11 +398,11 @@ __device__ __forceinline__ void gs_pair_row(const LevelView &L, const T *__restr
 			xo = (ry - ay) * ((T)1 / ac_o);
 		}
 		carry = __shfl(xz, 63, 64);
-		pE = doE; pO = doO; pZ = ext; pob = ob; pe = xe; po = xo; pz = xz;
+		pE = live; pO = doO; pZ = ext && last; pob = ob; pe = xe; po = xo; pz = xz;
 		if (last) break;
 	}
-	if (pE) st_row<T>(xr, pob, pe);
-	if (pO) st_row<T>(xr + 1, pob, po);
+	if (pO) { V2 v; v.x = pe; v.y = po; st_row<V2>(xr, pob, v); }
+	else if (pE) st_row<T>(xr, pob, pe);
 	if (pZ) st_row<T>(xr, pob + 2u * (uint32_t)sizeof(T), pz);
 }
 
@@ -523,10 +527,13 @@ __device__ __forceinline__ void gs_quad_row_f32(const LevelView &L, const float 
 				}
 			}
 		}
-		if (pE0) st_row<float>(xr, pob, v0);
-		if (pO1) st_row<float>(xr, pob + 4u, v1);
-		if (pE2) st_row<float>(xr, pob + 8u, v2);
-		if (pO3) st_row<float>(xr, pob + 12u, v3);
+		if (pO3) {
+			st_row<float4>(xr, pob, make_float4(v0, v1, v2, v3));
+		} else {
+			if (pE0) st_row<float>(xr, pob, v0);
+			if (pO1) st_row<float>(xr, pob + 4u, v1);
+			if (pE2) st_row<float>(xr, pob + 8u, v2);
+		}
 		if (pX) st_row<float>(xr, pob + 16u, v4);
 		float x0 = 0.0f, x2 = 0.0f, xx = 0.0f, y1 = 0.0f, y3 = 0.0f;
 		if (doE0) x0 = (r0 - e0) * (1.0f / c0);
@@ -550,15 +557,18 @@ __device__ __forceinline__ void gs_quad_row_f32(const LevelView &L, const float 
 			for (int q2 = 0; q2 < 12; q2++) o3 = o3 + p3[q2];
 			y3 = (r3 - o3) * (1.0f / c3);
 		}
-		pE0 = doE0; pE2 = doE2; pO1 = doO1; pO3 = doO3; pX = ext; pob = ob;
+		pE0 = live; pE2 = doE2; pO1 = doO1; pO3 = doO3; pX = ext && last; pob = ob;
 		v0 = x0; v1 = y1; v2 = x2; v3 = y3; v4 = xx;
 		if (last) break;
 		carry = __shfl(xx, 63, 64);
 	}
-	if (pE0) st_row<float>(xr, pob, v0);
-	if (pO1) st_row<float>(xr, pob + 4u, v1);
-	if (pE2) st_row<float>(xr, pob + 8u, v2);
-	if (pO3) st_row<float>(xr, pob + 12u, v3);
+	if (pO3) {
+		st_row<float4>(xr, pob, make_float4(v0, v1, v2, v3));
+	} else {
+		if (pE0) st_row<float>(xr, pob, v0);
+		if (pO1) st_row<float>(xr, pob + 4u, v1);
+		if (pE2) st_row<float>(xr, pob + 8u, v2);
+	}
 	if (pX) st_row<float>(xr, pob + 16u, v4);
 }
 
