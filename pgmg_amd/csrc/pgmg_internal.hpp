@@ -356,8 +356,8 @@ int launch_pair_sum(hipStream_t s, const LevelView &L, const double *a, const do
 // The block sums of launch_pair_sum(diff = 1) with `ext` point-major
 // (i + m*(j + n*k)) rather than in the level layout; returns the count.
 int launch_diff2_compact(hipStream_t s, const LevelView &L, const double *ext, const double *x, double *partial);
-// out[0] = sum of partial[0..n) in a fixed order.
-void launch_reduce(hipStream_t s, const double *partial, int n, double *out);
+// out[0] = sum of partial[0..n) in a fixed order; with flag, out[1] = *flag.
+void launch_reduce(hipStream_t s, const double *partial, int n, double *out, const double *flag = nullptr);
 // partial sums of r^2 (rhs_l2norm); returns count.
 template <typename T> int launch_sumsq(hipStream_t s, const LevelView &L, const T *r, double *partial);
 // rc = R res (gather form of the reference's scatter), xc = 0.

@@ -2579,22 +2579,29 @@ int launch_diff2_compact(hipStream_t s, const LevelView &L, const double *ext, c
 }
 
 // Fixed-order reduction: thread t sums partial[t], partial[t+1024], ... in
-// order, then a fixed binary tree.
-__global__ __launch_bounds__(1024) void k_reduce(const double *__restrict__ partial, int n, double *__restrict__ out) {
+// order, then a fixed binary tree, its last six levels within a wavefront.
+__global__ __launch_bounds__(1024) void k_reduce(const double *__restrict__ partial, int n, double *__restrict__ out,
+						 const double *__restrict__ flag) {
 	__shared__ double red[1024];
 	double s = 0.0;
 	for (int q = threadIdx.x; q < n; q += 1024) s = s + partial[q];
 	red[threadIdx.x] = s;
 	__syncthreads();
-	for (int w = 512; w > 0; w >>= 1) {
+	for (int w = 512; w >= 64; w >>= 1) {
 		if ((int)threadIdx.x < w) red[threadIdx.x] = red[threadIdx.x] + red[threadIdx.x + w];
 		__syncthreads();
 	}
-	if (threadIdx.x == 0) out[0] = red[0];
+	if (threadIdx.x >= 64) return;
+	s = red[threadIdx.x];
+	for (int w = 32; w > 0; w >>= 1) s = s + __shfl_down(s, w, 64);
+	if (threadIdx.x == 0) {
+		out[0] = s;
+		if (flag) out[1] = *flag;
+	}
 }
 
-void launch_reduce(hipStream_t s, const double *partial, int n, double *out) {
-	hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, s, partial, n, out);
+void launch_reduce(hipStream_t s, const double *partial, int n, double *out, const double *flag) {
+	hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, s, partial, n, out, flag);
 	HIPCHECK_LAUNCH();
 }
 
