@@ -394,11 +394,11 @@ void op_gs(pgmg_hier *h, int level, int mode, int nsweeps, XStart from = X_LEVEL
 					launch_gs_pair<T>(h->stream, L.v, lA<T>(L), lx<T>(L), lr<T>(L), q, fz);
 				}
 			} else {
-				// backward: colours 7..0
-				for (int c = 7; c >= 0; c--) {
-					const int ci = c & 1, cj = (c >> 1) & 1, ck = c >> 2;
-					ProfScope ps(h, KC_GS, level, (long long)((L.v.m - ci + 1) / 2) * ((L.v.n - cj + 1) / 2) * ((L.v.o - ck + 1) / 2));
-					launch_gs_colour<T>(h->stream, L.v, lA<T>(L), lx<T>(L), lr<T>(L), c);
+				// backward: colour pairs (7,6), (5,4), (3,2), (1,0)
+				for (int q = 3; q >= 0; q--) {
+					const int cj = q & 1, ck = q >> 1;
+					ProfScope ps(h, KC_GS, level, (long long)L.v.m * ((L.v.n - cj + 1) / 2) * ((L.v.o - ck + 1) / 2));
+					launch_gs_pair_back<T>(h->stream, L.v, lA<T>(L), lx<T>(L), lr<T>(L), q);
 				}
 			}
 		}

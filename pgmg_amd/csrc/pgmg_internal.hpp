@@ -302,6 +302,9 @@ template <typename T> void launch_gs_colour(hipStream_t s, const LevelView &L, c
 // x need not be cleared beforehand.
 template <typename T> void launch_gs_pair(hipStream_t s, const LevelView &L, const T *A, T *x, const T *r, int pair,
 					  bool from_zero = false);
+// Gauss-Seidel of the two colour classes (1,cj,ck) then (0,cj,ck): a pair of
+// the backward sweep.
+template <typename T> void launch_gs_pair_back(hipStream_t s, const LevelView &L, const T *A, T *x, const T *r, int pair);
 // One forward eight-colour sweep of a small level (gs_tile_ok) in one launch:
 // xout = the sweep of xin, which may be null for an x of zeros.  xin and xout
 // are different arrays in L's layout; only grid points of them are accessed.

@@ -984,6 +984,103 @@ __device__ __forceinline__ void gs_wave(const LevelView &L, const T *__restrict_
 	}
 }
 
+// Colour classes (1,cj,ck) and then (0,cj,ck), the backward sweep's order, of
+// one grid row by one wavefront, the odd points first.  Lane l holds the pair
+// (i0, i0+1), i0 = s0 + 2l; an even point's new odd neighbours are the lane's
+// own and the lane before's (shuffle; lane 0's is handed over by the segment
+// before, which is complete by then: an odd point reads only old even
+// points).  Next to the grid x is the halo's, zero or ghosts, as memory holds
+// it.  Arithmetic and order as in gs_point.
+//
+// Bound by bytes: one launch a class read every line of the coefficients
+// twice, half of it each time.  161x130x147 FP64, 27 points: 86 us for two
+// classes, 42 for the pair (4.2 TB/s).
+template <typename T, bool X>
+__device__ __forceinline__ void gs_pair_row_back(const LevelView &L, const T *__restrict__ A, T *__restrict__ x,
+						 const T *__restrict__ r, int j, int k) {
+	typedef typename Vec2<T>::type V2;
+	const int lane = threadIdx.x;
+	const long long row = idx3(L, 0, j, k);
+	const long long px = L.px, pxy = L.pxy, pa = L.pa;
+	const T *Ar = A + arow0(L, j, k);
+	const T *rr_ = r + row;
+	T *xr = x + row;
+	T carry = (T)0;
+	for (int s0 = 0; s0 < L.m; s0 += 128) {
+		const int i0 = s0 + 2 * lane;
+		const bool live = i0 < L.m, doO = i0 + 1 < L.m;
+		const uint32_t ob = (uint32_t)i0 * (uint32_t)sizeof(T);
+		T ax = (T)0, ay = (T)0, ac_e = (T)1, ac_o = (T)1, a12 = (T)0, a14 = (T)0;
+		T rx = (T)0, ry = (T)0, left = (T)0, right = (T)0;
+		T prod[12];
+		if (live) {
+			const V2 rr = ld_stream<V2>(rr_, ob);
+			rx = rr.x; ry = rr.y;
+#pragma unroll
+			for (int rq = 0; rq < 9; rq++) {
+				const T *xq = xr + (rq % 3 - 1) * px + (rq / 3 - 1) * pxy;
+				const V2 am = coef_or_zero<V2, X>(Ar, 3 * rq, pa, ob);
+				const V2 a0 = coef_or_zero<V2, X>(Ar, 3 * rq + 1, pa, ob);
+				const V2 ap = coef_or_zero<V2, X>(Ar, 3 * rq + 2, pa, ob);
+				const V2 xv = ld_row<V2>(xq, ob);
+				const T xm = ld_row<T>(xq - 1, ob);
+				const T xp = doO ? ld_row<T>(xq + 2, ob) : (T)0;
+				ay = ay + am.y * xv.x;
+				if (rq == 4) ac_o = a0.y;
+				else ay = ay + a0.y * xv.y;
+				ay = ay + ap.y * xp;
+				if (rq < 4) {
+					ax = ax + am.x * xm;
+					ax = ax + a0.x * xv.x;
+					ax = ax + ap.x * xv.y;
+				} else if (rq == 4) {
+					ac_e = a0.x; a12 = am.x; a14 = ap.x;
+					left = xm;
+					right = xv.y;
+				} else {
+					prod[3 * (rq - 5)] = am.x * xm;
+					prod[3 * (rq - 5) + 1] = a0.x * xv.x;
+					prod[3 * (rq - 5) + 2] = ap.x * xv.y;
+				}
+			}
+		}
+		T xo = (T)0;
+		if (doO) xo = (ry - ay) * ((T)1 / ac_o);
+		// with every lane active
+		const T before = __shfl_up(xo, 1, 64);
+		if (lane > 0) left = before;
+		else if (s0 > 0) left = carry;
+		if (doO) right = xo;
+		carry = __shfl(xo, 63, 64);
+		if (live) {
+			ax = ax + a12 * left;
+			ax = ax + a14 * right;
+#pragma unroll
+			for (int q = 0; q < 12; q++) ax = ax + prod[q];
+			const T xe = (rx - ax) * ((T)1 / ac_e);
+			if (doO) { V2 v; v.x = xe; v.y = xo; st_row<V2>(xr, ob, v); }
+			else st_row<T>(xr, ob, xe);
+		}
+	}
+}
+
+template <typename T, bool X>
+__global__ __launch_bounds__(64) void k_gs_pair_back(LevelView L, const T *__restrict__ A, T *__restrict__ x,
+						     const T *__restrict__ r, int cj, int ck) {
+	const int w = xcd_block((int)blockIdx.x, (int)gridDim.x), nb = (L.n - cj + 1) >> 1;
+	gs_pair_row_back<T, X>(L, A, x, r, 2 * (w % nb) + cj, 2 * (w / nb) + ck);
+}
+
+template <typename T>
+void launch_gs_pair_back(hipStream_t s, const LevelView &L, const T *A, T *x, const T *r, int pair) {
+	const int cj = pair & 1, ck = (pair >> 1) & 1;
+	const int nb = (L.n - cj + 1) >> 1, nd = (L.o - ck + 1) >> 1;
+	if (nb <= 0 || nd <= 0) return;
+	if (L.cross) hipLaunchKernelGGL((k_gs_pair_back<T, true>), dim3(nb * nd), dim3(64), 0, s, L, A, x, r, cj, ck);
+	else hipLaunchKernelGGL((k_gs_pair_back<T, false>), dim3(nb * nd), dim3(64), 0, s, L, A, x, r, cj, ck);
+	HIPCHECK_LAUNCH();
+}
+
 template <typename T, bool Z, bool X>
 __global__ __launch_bounds__(256) void k_gs_pair(LevelView L, const T *__restrict__ A, T *__restrict__ x,
 						 const T *__restrict__ r, int cj, int ck) {
@@ -4429,6 +4526,7 @@ void launch_b_add_x(hipStream_t s, const SlotDev *slots, WorkList wl, int chunk)
 // ------------------------------------------------------ instantiations
 #define INST(T) \
 	template void launch_gs_colour<T>(hipStream_t, const LevelView &, const T *, T *, const T *, int); \
+	template void launch_gs_pair_back<T>(hipStream_t, const LevelView &, const T *, T *, const T *, int); \
 	template void launch_gs_pair<T>(hipStream_t, const LevelView &, const T *, T *, const T *, int, bool); \
 	template void launch_gs_plane<T>(hipStream_t, const LevelView &, const T *, T *, const T *, int); \
 	template void launch_gs_planes<T>(hipStream_t, const LevelView &, const T *, T *, const T *, int); \
