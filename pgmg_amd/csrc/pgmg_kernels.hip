@@ -3617,69 +3617,91 @@ void launch_lu_assemble(hipStream_t s, const LevelView &L, const double *A, doub
 	HIPCHECK_LAUNCH();
 }
 
+// The half width of the band of L's bottom operator, and N where it has none.
+__host__ __device__ inline int lu_band(const LevelView &L, int N) {
+	return L.prd ? N : min(N, 1 + L.m + L.m * L.n);
+}
+
 // Right-looking LU with partial pivoting by one workgroup: pivot = first
 // row of largest modulus (dgetrf's rule, region_tr.cc:518), column scaled
 // by the pivot's reciprocal, rank-1 update.  info = first zero pivot (1-based)
 // and info[1] = 1 when the factor fails the test of region_tr.cc:526-533.
-__global__ __launch_bounds__(1024) void k_lu_factor(int N, double *__restrict__ LU, int *__restrict__ ipiv,
+//
+// Only the operator's band is worked on (half width `band`; N: none): column
+// c has nothing below row c + band, whatever was interchanged before, and
+// with interchanges row c ends at column c + 2 band; what is left out are
+// updates by 0 (an operator with infinities or NaN aside).  A wavefront updates
+// four columns at a time, a lane a row.  11x7x9 unknowns: 33 ms over the whole
+// matrix with one entry a thread and a 64-bit division for each, 5.1 so.  The largest entry is found with one barrier: within each wavefront,
+// then by every wavefront from the 16 that remain.
+__global__ __launch_bounds__(1024) void k_lu_factor(int N, int band, double *__restrict__ LU, int *__restrict__ ipiv,
 						    int *__restrict__ info) {
-	__shared__ double bv[1024];
-	__shared__ int bi[1024];
-	__shared__ int s_piv, s_info, s_nz;
+	__shared__ double bv[16];
+	__shared__ int bi[16];
+	__shared__ int s_info;
 	const int tid = threadIdx.x, nt = blockDim.x;
+	const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	if (tid == 0) s_info = 0;
+	__syncthreads();
+	// the larger entry, of equal ones the first
+	const auto better = [](double v, int r, double &best, int &at) {
+		if (v > best || (v == best && r < at)) { best = v; at = r; }
+	};
 	for (int c = 0; c < N; c++) {
+		const int rend = min(N, c + band + 1), cend = min(N, c + 2 * band + 1);
+		double *const Lc = LU + (long long)c * N;
 		double best = -1.0;
-		int bidx = N;
-		for (int r = c + tid; r < N; r += nt) {
-			const double v = fabs(LU[r + (long long)c * N]);
-			if (v > best) { best = v; bidx = r; }
+		int at = N;
+		for (int r = c + tid; r < rend; r += nt) {
+			const double v = fabs(Lc[r]);
+			if (v > best) { best = v; at = r; }
 		}
-		bv[tid] = best; bi[tid] = bidx;
+		for (int w = 32; w > 0; w >>= 1) better(__shfl_xor(best, w, 64), __shfl_xor(at, w, 64), best, at);
+		if (lane == 0) { bv[wave] = best; bi[wave] = at; }
 		__syncthreads();
-		for (int w = nt / 2; w > 0; w >>= 1) {
-			if (tid < w) {
-				const double ov = bv[tid + w];
-				const int oi = bi[tid + w];
-				if (ov > bv[tid] || (ov == bv[tid] && oi < bi[tid])) { bv[tid] = ov; bi[tid] = oi; }
-			}
-			__syncthreads();
-		}
-		if (tid == 0) {
-			// The sequential rule keeps the diagonal unless another entry
-			// is strictly larger; a NaN column keeps the diagonal.
-			int piv = bi[0];
-			if (!(bv[0] > fabs(LU[c + (long long)c * N])) || piv >= N) piv = c;
-			s_piv = piv;
-			s_nz = LU[piv + (long long)c * N] != 0.0;
-			ipiv[c] = piv;
-		}
+		best = bv[lane & 15];
+		at = bi[lane & 15];
+		for (int w = 8; w > 0; w >>= 1) better(__shfl_xor(best, w, 64), __shfl_xor(at, w, 64), best, at);
+		// The sequential rule keeps the diagonal unless another entry is
+		// strictly larger; a NaN column keeps the diagonal.  Every thread
+		// reads the same two entries before any is changed.
+		int piv = at;
+		const double diag = Lc[c];
+		if (!(best > fabs(diag)) || piv >= N) piv = c;
+		const double pivot = Lc[piv];
+		const bool nz = pivot != 0.0;
 		__syncthreads();
-		const int piv = s_piv;
-		// Read once by thread 0 before any swap, so every thread takes the
-		// same branch and reaches the same barriers.
-		const bool nz = s_nz != 0;
+		if (tid == 0) ipiv[c] = piv;
 		if (nz) {
 			if (piv != c) {
 				for (int jcol = tid; jcol < N; jcol += nt) {
-					const double t = LU[c + (long long)jcol * N];
-					LU[c + (long long)jcol * N] = LU[piv + (long long)jcol * N];
-					LU[piv + (long long)jcol * N] = t;
+					double *const col = LU + (long long)jcol * N;
+					const double t = col[c];
+					col[c] = col[piv];
+					col[piv] = t;
 				}
+				__syncthreads();
 			}
-			__syncthreads();
-			const double rp = 1.0 / LU[c + (long long)c * N];
-			for (int r = c + 1 + tid; r < N; r += nt) LU[r + (long long)c * N] *= rp;
+			const double rp = 1.0 / pivot;
+			for (int r = c + 1 + tid; r < rend; r += nt) Lc[r] *= rp;
 		} else if (tid == 0 && s_info == 0) {
 			s_info = c + 1;
 		}
 		__syncthreads();
-		const int rem = N - c - 1;
-		const long long tot = (long long)rem * rem;
-		for (long long q = tid; q < tot; q += nt) {
-			const int r = c + 1 + (int)(q % rem), jcol = c + 1 + (int)(q / rem);
-			const double u = LU[c + (long long)jcol * N];
-			if (u != 0.0) LU[r + (long long)jcol * N] -= LU[r + (long long)c * N] * u;
+		// four columns at once, their loads together
+		for (int j0 = c + 1 + 4 * wave; j0 < cend; j0 += 4 * (nt / 64)) {
+			double u[4];
+#pragma unroll
+			for (int q = 0; q < 4; q++) u[q] = j0 + q < cend ? LU[(long long)(j0 + q) * N + c] : 0.0;
+			for (int r = c + 1 + lane; r < rend; r += 64) {
+				const double l = Lc[r];
+				double v[4];
+#pragma unroll
+				for (int q = 0; q < 4; q++) v[q] = LU[(long long)min(j0 + q, cend - 1) * N + r];
+#pragma unroll
+				for (int q = 0; q < 4; q++)
+					if (u[q] != 0.0) LU[(long long)(j0 + q) * N + r] = v[q] - l * u[q];
+			}
 		}
 		__syncthreads();
 	}
@@ -3690,8 +3712,9 @@ __global__ __launch_bounds__(1024) void k_lu_factor(int N, double *__restrict__ 
 	}
 }
 
-void launch_lu_factor(hipStream_t s, int N, double *LU, int *ipiv, int *info) {
-	hipLaunchKernelGGL(k_lu_factor, dim3(1), dim3(1024), 0, s, N, LU, ipiv, info);
+void launch_lu_factor(hipStream_t s, const LevelView &L, double *LU, int *ipiv, int *info) {
+	const int N = L.m * L.n * L.o;
+	hipLaunchKernelGGL(k_lu_factor, dim3(1), dim3(1024), 0, s, N, lu_band(L, N), LU, ipiv, info);
 	HIPCHECK_LAUNCH();
 }
 
@@ -3716,11 +3739,6 @@ void launch_lu_factor(hipStream_t s, int N, double *LU, int *ipiv, int *info) {
 // four wavefronts of twice the registers).
 const int kLuWaves = 8;
 const int kLuMax = 2048;  // enable_exact takes fewer points than this
-
-// The half width of the band of L's bottom operator, and N where it has none.
-__device__ __forceinline__ int lu_band(const LevelView &L, int N) {
-	return L.prd ? N : min(N, 1 + L.m + L.m * L.n);
-}
 
 // Correctly rounded n / d from y = 1/d rounded to nearest: the second
 // correction starts from a faithful quotient and its remainder is exact
