@@ -394,7 +394,7 @@ public:
 	~HostReadout();
 	// The grid points of d to out; out is complete on return.
 	hipError_t copy(hipStream_t s, const LevelView &L, const double *d, double *out);
-	static const int kSlots = 16;
+	static const int kSlots = 8;
 
 private:
 	std::mutex mu;
