@@ -2993,7 +2993,7 @@ __device__ __forceinline__ void restrict_any(const LevelView &F, const LevelView
 // The lone hierarchy restricts onto a coarse level of at least
 // kRestrictSplitPoints points in two launches: the coarse points whose eight
 // surrounding cubes are interior (restrict_interior, every lane on the same
-// path), and the shell of the others (restrict_point).  One launch over all
+// path), and the shell of the others (restrict_any).  One launch over all
 // points put a boundary point into a third of the wavefronts (I = 0 and the
 // last I), which then ran both paths: 257^3 -> 129^3 in FP32 87 us, split
 // 37 us; onto 65^3 30 -> 22 us; onto 33^3 the second launch cost more (18 ->
