@@ -3813,8 +3813,10 @@ void launch_lu_factor(hipStream_t s, const LevelView &L, double *LU, int *ipiv, 
 // R mod 8, which applies the columns to it 32 at a time: a column's unknown
 // is read out of a lane (v_readlane), the block's own columns form the chain,
 // and the coefficients of its next two pieces of work are in flight
-// meanwhile (one piece ahead: 138 us below).  One barrier per 32 columns.  Every row subtracts its terms one by one in column order,
-// as the column-by-column loop, so x is the same.
+// meanwhile (one piece ahead: 138 us below).  One barrier per 32 columns.
+// Every row subtracts its terms one by one in column order, as the
+// column-by-column loop, so x is the same; where it would not be, that loop is
+// run (lu_solve_columns).
 //
 // Without interchanges the factor keeps the operator's band (half width bw =
 // 1 + m + mn in the order of the points): blocks outside it, which are zero,
@@ -3960,34 +3962,10 @@ __device__ __forceinline__ void lu_back(const LuPiece &p, double *__restrict__ x
 	if (l < 32) xs[row] = l < 0 ? xr : sol;
 }
 
-template <typename T>
-__device__ __forceinline__ void lu_solve_body(const LevelView &L, int N, const double *__restrict__ LU,
-					      const int *__restrict__ ipiv, const T *__restrict__ r, T *__restrict__ x) {
-	__shared__ double xs[kLuMax];
-	__shared__ int sp[kLuMax];
-	const int tid = threadIdx.x, nt = blockDim.x;
-	const int w = __builtin_amdgcn_readfirstlane(tid / 64);
-	const int nblk = (N + 63) / 64, ncb = 2 * nblk;
-	int moved = 0;
-	for (int q = tid; q < 64 * nblk; q += nt) {
-		double v = 0.0;
-		if (q < N) {
-			const int i = q % L.m, j = (q / L.m) % L.n, k = q / (L.m * L.n);
-			v = (double)r[idx3(L, i, j, k)];
-			sp[q] = ipiv[q];
-			moved |= sp[q] != q;
-		}
-		xs[q] = v;
-	}
-	moved = __syncthreads_or(moved);
-	if (moved) {
-		if (tid == 0)
-			for (int c = 0; c < N; c++) {
-				const int p = sp[c];
-				if (p != c) { const double t = xs[c]; xs[c] = xs[p]; xs[p] = t; }
-			}
-		__syncthreads();
-	}
+// The substitutions by pieces; xs ends with 0 past the end.
+__device__ __forceinline__ void lu_solve_pieces(const LevelView &L, int N, const double *__restrict__ LU,
+						double *__restrict__ xs, int w, int nblk, int ncb, int moved) {
+	const int tid = threadIdx.x;
 	const int band = lu_band(L, N);
 	const int bl = moved ? N : band, bu = moved ? min(N, 2 * band) : band;
 	LuPiece p0, p1, p2;
@@ -4035,6 +4013,123 @@ __device__ __forceinline__ void lu_solve_body(const LevelView &L, int N, const d
 		for (; passed < ncb; passed++) __syncthreads();
 	}
 	__syncthreads();
+}
+
+// |v| of an infinity or NaN is not at most this.
+const double kLargest = 1.7976931348623157e308;
+
+// The substitutions column by column over the whole factor, unknowns of 0
+// skipped, for the two kinds of source whose bits the pieces do not keep: one
+// that holds a -0 (the pieces subtract a term of 0 where this skips it, and
+// -0 - -0 is 0; no other source comes to a -0 before a quotient), and one with
+// an unknown that is not finite (whose terms of 0 the pieces drop outside the
+// band and form within a block).  The pieces leave a row not finite where an
+// unknown of it, or a factor's entry it takes, is not, so their solution tells
+// the second kind where the source does not.
+//
+// R rows a thread, in registers, with the next column's entries of them in
+// flight, one barrier a column: 11x7x9 unknowns 372 us, 4x4x4 25 (by pieces 109
+// and 14; rows in LDS, as every source was solved before the pieces, 475 and 43).
+template <int R>
+__device__ __forceinline__ void lu_solve_columns(int N, const double *__restrict__ LU, double *__restrict__ xs) {
+	const int nt = 64 * kLuWaves;
+	double xr[R], a[R];
+	int row[R], at[R];
+#pragma unroll
+	for (int q = 0; q < R; q++) {
+		row[q] = (int)threadIdx.x + q * nt;
+		at[q] = min(row[q], N - 1);
+		xr[q] = xs[at[q]];
+		a[q] = LU[at[q]];
+	}
+	for (int c = 0; c < N - 1; c++) {  // the last column has no rows below
+		const double *const next = LU + (long long)(c + 1) * N;
+#pragma unroll
+		for (int q = 0; q < R; q++)
+			if (row[q] == c) xs[c] = xr[q];
+		double b[R];
+#pragma unroll
+		for (int q = 0; q < R; q++) b[q] = next[at[q]];
+		__syncthreads();
+		const double v = xs[c];
+		if (v != 0.0) {
+#pragma unroll
+			for (int q = 0; q < R; q++) xr[q] = row[q] > c ? xr[q] - v * a[q] : xr[q];
+		}
+#pragma unroll
+		for (int q = 0; q < R; q++) a[q] = b[q];
+	}
+	// a holds the last column
+	for (int c = N - 1; c >= 0; c--) {
+		const double *const next = LU + (long long)max(c - 1, 0) * N;
+#pragma unroll
+		for (int q = 0; q < R; q++)
+			if (row[q] == c) xs[c] = xr[q] / a[q];
+		double b[R];
+#pragma unroll
+		for (int q = 0; q < R; q++) b[q] = next[at[q]];
+		__syncthreads();
+		const double v = xs[c];
+		if (v != 0.0) {
+#pragma unroll
+			for (int q = 0; q < R; q++) xr[q] = row[q] < c ? xr[q] - v * a[q] : xr[q];
+		}
+#pragma unroll
+		for (int q = 0; q < R; q++) a[q] = b[q];
+	}
+	__syncthreads();
+}
+
+template <typename T>
+__device__ __forceinline__ void lu_solve_body(const LevelView &L, int N, const double *__restrict__ LU,
+					      const int *__restrict__ ipiv, const T *__restrict__ r, T *__restrict__ x) {
+	__shared__ double xs[kLuMax];
+	__shared__ int sp[kLuMax];
+	const int tid = threadIdx.x, nt = blockDim.x;
+	const int w = __builtin_amdgcn_readfirstlane(tid / 64);
+	const int nblk = (N + 63) / 64, ncb = 2 * nblk;
+	int moved = 0, columns = 0;
+	for (int q = tid; q < N; q += nt) {
+		sp[q] = ipiv[q];
+		moved |= sp[q] != q;
+	}
+	// the source into xs, interchanged; whether it is one for the columns
+	const auto load = [&] {
+		int other = 0;
+		for (int q = tid; q < 64 * nblk; q += nt) {
+			double v = 0.0;
+			if (q < N) {
+				const int i = q % L.m, j = (q / L.m) % L.n, k = q / (L.m * L.n);
+				v = (double)r[idx3(L, i, j, k)];
+				other |= !(fabs(v) <= kLargest) || (v == 0.0 && __double_as_longlong(v) != 0);
+			}
+			xs[q] = v;
+		}
+		other = __syncthreads_or(other);
+		moved = __syncthreads_or(moved);
+		if (moved) {
+			if (tid == 0)
+				for (int c = 0; c < N; c++) {
+					const int p = sp[c];
+					if (p != c) { const double t = xs[c]; xs[c] = xs[p]; xs[p] = t; }
+				}
+			__syncthreads();
+		}
+		return other;
+	};
+	columns = load();
+	if (!columns) {
+		lu_solve_pieces(L, N, LU, xs, w, nblk, ncb, moved);
+		int bad = 0;
+		for (int q = tid; q < N; q += nt) bad |= !(fabs(xs[q]) <= kLargest);
+		columns = __syncthreads_or(bad);
+		if (columns) load();
+	}
+	if (columns) {
+		if (N <= 64 * kLuWaves) lu_solve_columns<1>(N, LU, xs);
+		else if (N <= 128 * kLuWaves) lu_solve_columns<2>(N, LU, xs);
+		else lu_solve_columns<kLuMax / (64 * kLuWaves)>(N, LU, xs);
+	}
 	for (int q = tid; q < N; q += nt) {
 		const int i = q % L.m, j = (q / L.m) % L.n, k = q / (L.m * L.n);
 		x[idx3(L, i, j, k)] = (T)xs[q];
