@@ -528,7 +528,7 @@ int slot_setup(pgmg_batch *b, int s, const pgmg_dims *d, int family, uint64_t se
 	for (int l = 1; l < S.nl; l++) launch_rat(st, D.lv[l - 1], D.lv[l], D.A[l - 1], D.A[l]);
 	if (S.want_lu) {
 		launch_lu_assemble(st, D.lv[bl], D.A[bl], D.LU);
-		launch_lu_factor(st, D.lv[bl], D.LU, D.ipiv, b->d_info + 2 * s);
+		launch_lu_factor(st, D.lv[bl], D.A[bl], D.LU, D.ipiv, b->d_info + 2 * s);
 	}
 	if (b->mixed)
 		for (int l = 0; l < S.nl; l++) launch_round_f32(st, D.A[l], D.A32[l], 27 * D.lv[l].npad);

@@ -778,7 +778,7 @@ static int factor_bottom(pgmg_hier *h) {
 	h->lu_N = (int)N;
 	launch_fill<double>(h->stream, h->LU, N * N, 0.0);
 	launch_lu_assemble(h->stream, B.v, B.A, h->LU);
-	launch_lu_factor(h->stream, B.v, h->LU, h->ipiv, h->lu_info);
+	launch_lu_factor(h->stream, B.v, B.A, h->LU, h->ipiv, h->lu_info);
 	int info[2] = {0, 1};
 	HIP_TRY(hipMemcpyAsync(info, h->lu_info, sizeof(info), hipMemcpyDeviceToHost, h->stream));
 	HIP_TRY(hipStreamSynchronize(h->stream));

@@ -372,7 +372,8 @@ template <typename T> void launch_interp(hipStream_t s, const LevelView &C, cons
 void launch_rat(hipStream_t s, const LevelView &F, const LevelView &C, const double *Af, double *Ac);
 // Dense bottom LU.
 void launch_lu_assemble(hipStream_t s, const LevelView &L, const double *A, double *LU);
-void launch_lu_factor(hipStream_t s, const LevelView &L, double *LU, int *ipiv, int *info);
+// LU holds L's assembled operator A; the factor is left in its place.
+void launch_lu_factor(hipStream_t s, const LevelView &L, const double *A, double *LU, int *ipiv, int *info);
 template <typename T> void launch_lu_solve(hipStream_t s, const LevelView &L, int N, const double *LU, const int *ipiv,
 					   const T *r, T *x);
 // Problem generation on the device.

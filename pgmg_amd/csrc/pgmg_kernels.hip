@@ -3659,17 +3659,20 @@ void launch_rat(hipStream_t s, const LevelView &F, const LevelView &C, const dou
 // ---------------------------------------------------------- bottom LU
 
 // Dense column-major matrix of the bottom level, row = point, column =
-// neighbour (region_tr.cc:486-504).  The caller zero-fills LU first.
-__global__ void k_lu_assemble(LevelView L, const double *__restrict__ A, double *__restrict__ LU) {
+// neighbour (region_tr.cc:486-504): entry t of the N * 27.  LU is zero before.
+__device__ __forceinline__ void lu_assemble_entry(const LevelView &L, const double *__restrict__ A, double *__restrict__ LU,
+						  long long t) {
 	const int N = L.m * L.n * L.o;
-	const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (tid >= (long long)N * 27) return;
-	const int e = (int)(tid % 27), p = (int)(tid / 27);
+	const int e = (int)(t % 27), p = (int)(t / 27);
 	const int i = p % L.m, j = (p / L.m) % L.n, k = p / (L.m * L.n);
 	const int qi = i + e % 3 - 1, qj = j + (e / 3) % 3 - 1, qk = k + e / 9 - 1;
 	if (qi < 0 || qi >= L.m || qj < 0 || qj >= L.n || qk < 0 || qk >= L.o) return;
 	const int q = qi + L.m * (qj + L.n * qk);
 	LU[p + (long long)q * N] = A[aidx3(L, e, i, j, k)];
+}
+__global__ void k_lu_assemble(LevelView L, const double *__restrict__ A, double *__restrict__ LU) {
+	const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+	if (t < (long long)L.m * L.n * L.o * 27) lu_assemble_entry(L, A, LU, t);
 }
 
 // With periodic axes, one thread per row: a wrapped neighbour's column is its
@@ -3703,6 +3706,9 @@ void launch_lu_assemble(hipStream_t s, const LevelView &L, const double *A, doub
 	HIPCHECK_LAUNCH();
 }
 
+// |v| of an infinity or NaN is not at most this.
+const double kLargest = 1.7976931348623157e308;
+
 // The half width of the band of L's bottom operator, and N where it has none.
 __host__ __device__ inline int lu_band(const LevelView &L, int N) {
 	return L.prd ? N : min(N, 1 + L.m + L.m * L.n);
@@ -3716,15 +3722,18 @@ __host__ __device__ inline int lu_band(const LevelView &L, int N) {
 // Only the operator's band is worked on (half width `band`; N: none): column
 // c has nothing below row c + band, whatever was interchanged before, and
 // with interchanges row c ends at column c + 2 band; what is left out are
-// updates by 0 (an operator with infinities or NaN aside).  A wavefront updates
-// four columns at a time, a lane a row.  11x7x9 unknowns: 33 ms over the whole
-// matrix with one entry a thread and a 64-bit division for each, 5.1 so.  The largest entry is found with one barrier: within each wavefront,
-// then by every wavefront from the 16 that remain.
-__global__ __launch_bounds__(1024) void k_lu_factor(int N, int band, double *__restrict__ LU, int *__restrict__ ipiv,
-						    int *__restrict__ info) {
+// updates by 0.  (L's zeros below the band still take the pivot's sign.)  A
+// wavefront updates four columns at a time, a lane a row.  11x7x9 unknowns:
+// 33 ms over the whole matrix with one entry a thread and a 64-bit division for
+// each, 5.1 so.  The largest entry is found with one barrier: within each
+// wavefront, then by every wavefront from the 16 that remain.
+//
+// Returns whether this thread met an entry that is not finite: 0 times that is
+// NaN, so what was left out is not 0 then.
+__device__ __forceinline__ bool lu_factor_pass(int N, int band, double *__restrict__ LU, int *__restrict__ ipiv, int &s_info) {
 	__shared__ double bv[16];
 	__shared__ int bi[16];
-	__shared__ int s_info;
+	bool odd = false;
 	const int tid = threadIdx.x, nt = blockDim.x;
 	const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	if (tid == 0) s_info = 0;
@@ -3769,7 +3778,11 @@ __global__ __launch_bounds__(1024) void k_lu_factor(int N, int band, double *__r
 				__syncthreads();
 			}
 			const double rp = 1.0 / pivot;
-			for (int r = c + 1 + tid; r < rend; r += nt) Lc[r] *= rp;
+			for (int r = c + 1 + tid; r < N; r += nt) {
+				const double l = Lc[r] * rp;
+				Lc[r] = l;
+				odd |= !(fabs(l) <= kLargest);
+			}
 		} else if (tid == 0 && s_info == 0) {
 			s_info = c + 1;
 		}
@@ -3778,7 +3791,10 @@ __global__ __launch_bounds__(1024) void k_lu_factor(int N, int band, double *__r
 		for (int j0 = c + 1 + 4 * wave; j0 < cend; j0 += 4 * (nt / 64)) {
 			double u[4];
 #pragma unroll
-			for (int q = 0; q < 4; q++) u[q] = j0 + q < cend ? LU[(long long)(j0 + q) * N + c] : 0.0;
+			for (int q = 0; q < 4; q++) {
+				u[q] = j0 + q < cend ? LU[(long long)(j0 + q) * N + c] : 0.0;
+				odd |= !(fabs(u[q]) <= kLargest);
+			}
 			for (int r = c + 1 + lane; r < rend; r += 64) {
 				const double l = Lc[r];
 				double v[4];
@@ -3791,6 +3807,25 @@ __global__ __launch_bounds__(1024) void k_lu_factor(int N, int band, double *__r
 		}
 		__syncthreads();
 	}
+	return odd;
+}
+
+// A factor in which the band met an infinity or a NaN is made again, from the
+// operator, over the whole matrix, where such an entry reaches rows below the
+// band (11x7x9 unknowns 24.7 ms, 5.4 without).
+__global__ __launch_bounds__(1024) void k_lu_factor(LevelView L, const double *__restrict__ A, int N,
+						    double *__restrict__ LU, int *__restrict__ ipiv, int *__restrict__ info) {
+	__shared__ int s_info;
+	const int tid = threadIdx.x, nt = blockDim.x;
+	for (int band = lu_band(L, N);;) {
+		const bool odd = lu_factor_pass(N, band, LU, ipiv, s_info);
+		if (!__syncthreads_or(odd) || band >= N) break;
+		for (long long q = tid; q < (long long)N * N; q += nt) LU[q] = 0.0;
+		__syncthreads();
+		for (long long t = tid; t < 27LL * N; t += nt) lu_assemble_entry(L, A, LU, t);
+		__syncthreads();
+		band = N;
+	}
 	if (tid == 0) {
 		info[0] = s_info;
 		const double hi = fabs(LU[0]), lo = fabs(LU[(long long)N * N - 1]);
@@ -3798,9 +3833,8 @@ __global__ __launch_bounds__(1024) void k_lu_factor(int N, int band, double *__r
 	}
 }
 
-void launch_lu_factor(hipStream_t s, const LevelView &L, double *LU, int *ipiv, int *info) {
-	const int N = L.m * L.n * L.o;
-	hipLaunchKernelGGL(k_lu_factor, dim3(1), dim3(1024), 0, s, N, lu_band(L, N), LU, ipiv, info);
+void launch_lu_factor(hipStream_t s, const LevelView &L, const double *A, double *LU, int *ipiv, int *info) {
+	hipLaunchKernelGGL(k_lu_factor, dim3(1), dim3(1024), 0, s, L, A, L.m * L.n * L.o, LU, ipiv, info);
 	HIPCHECK_LAUNCH();
 }
 
@@ -4014,9 +4048,6 @@ __device__ __forceinline__ void lu_solve_pieces(const LevelView &L, int N, const
 	}
 	__syncthreads();
 }
-
-// |v| of an infinity or NaN is not at most this.
-const double kLargest = 1.7976931348623157e308;
 
 // The substitutions column by column over the whole factor, unknowns of 0
 // skipped, for the two kinds of source whose bits the pieces do not keep: one
