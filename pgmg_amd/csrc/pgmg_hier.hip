@@ -952,7 +952,7 @@ int pgmg_clear_x(pgmg_hier *h, int level) {
 	int rc = check_level(h, level);
 	if (rc) return rc;
 	launch_fill<double>(h->stream, h->lev[level].x, h->lev[level].v.npad, 0.0);
-	HIP_TRY(hipGetLastError());
+	HIP_TRY(hipStreamSynchronize(h->stream));
 	return PGMG_OK;
 }
 
