@@ -126,24 +126,32 @@ enum { L_TOP_ROWS = 0, L_X_TOP_ROWS, L_TOP_ONE, L_TOP_PTS, L_X_PAIR0, L_X_PAIR1,
 // per launch class, measured on the batch's own first steps.  Trial t
 // (t = 0 .. kTuneSteps-1, two rounds over the candidates) runs the launches
 // between two convergence checks with candidate t % kNumChunks, each
-// bracketed by timing events; each class then keeps the chunk with the
-// least time per work unit (the smaller of its rounds).  A unit's arithmetic
-// does not depend on the chunk, so the trial steps are ordinary steps with
-// the same results.  (Running the trials again whenever the active slots'
-// level-0 rows halved or doubled was tried on the 256-problem batch: 14.4 s
-// against 14.0 s, the trial steps costing more than the later choices
-// gained.)
+// bracketed by timing events.  A launch too short for a candidate (chunk_of) says
+// nothing of it: a candidate's time per work unit (the smaller of its rounds) is
+// that of the launches long enough for it, and is held against one unit a
+// workgroup on those; each class keeps the best, 1 where no launch was long
+// enough for more.  A unit's arithmetic does not depend on the chunk, so the
+// trial steps are ordinary steps with the same results.  (Running the trials
+// again whenever the active slots' level-0 rows halved or doubled was tried on
+// the 256-problem batch: 14.4 s against 14.0 s, the trial steps costing more
+// than the later choices gained.)
 enum { TC_PAIR = 0, TC_RES, TC_RESTOP, TC_RESTRICT, TC_INTERP, TC_ADD, TC_COUNT };
 const int kChunks[] = {1, 2, 4, 8};
 const int kNumChunks = 4;
 const int kTuneSteps = 2 * kNumChunks;
 
+// A launch keeps at least kMinGroups workgroups (four to a CU) where its units
+// allow: with fewer, units that could run side by side follow one another in a
+// workgroup (a trial of 8 units a workgroup took 65 us on levels of 40 units
+// that take 12 one by one).
+const int kMinGroups = 1024;
 struct TileTuner {
 	int step = 0;           // trial steps done
 	bool done = false;
 	int best[TC_COUNT] = {1, 1, 1, 1, 1, 1};
-	double ms[TC_COUNT][kNumChunks][2] = {};        // per candidate and round
-	long long units[TC_COUNT][kNumChunks][2] = {};
+	// per candidate and round, and one unit a workgroup on the same launches
+	struct Sum { double ms = 0; long long units = 0; };
+	Sum sum[TC_COUNT][kNumChunks][2], one[TC_COUNT][kNumChunks][2];
 	struct Mark { int cls, cand, round; long long units; hipEvent_t a, b; };
 	std::vector<Mark> marks;    // this step's timed launches
 	std::vector<hipEvent_t> pool;
@@ -281,11 +289,6 @@ int build_plan(pgmg_batch *b) {
 	return PGMG_OK;
 }
 
-// A launch keeps at least kMinGroups workgroups (four to a CU) where its units
-// allow: with fewer, units that could run side by side follow one another in a
-// workgroup (a trial of 8 units a workgroup took 65 us on levels of 40 units
-// that take 12 one by one).
-const int kMinGroups = 1024;
 int chunk_of(pgmg_batch *b, int cls, int units) {
 	const int c = b->tune.done ? b->tune.best[cls] : kChunks[b->tune.step % kNumChunks];
 	return std::max(1, std::min(c, units / kMinGroups));
@@ -298,7 +301,8 @@ void tuned(pgmg_batch *b, int cls, const WorkList &wl, F launch) {
 	if (wl.n <= 0) return;
 	const int c = chunk_of(b, cls, wl.total);
 	TileTuner &t = b->tune;
-	if (t.done) { launch(c); return; }
+	// only launches long enough for two units a workgroup and for the candidate
+	if (t.done || c != kChunks[t.step % kNumChunks] || wl.total < 2 * kMinGroups) { launch(c); return; }
 	if (t.used + 2 > t.pool.size()) {
 		for (int q = 0; q < 64; q++) {
 			hipEvent_t e;
@@ -323,23 +327,34 @@ void tune_collect(pgmg_batch *b) {
 	for (const auto &mk : t.marks) {
 		float ms = 0;
 		if (hipEventElapsedTime(&ms, mk.a, mk.b) == hipSuccess) {
-			t.ms[mk.cls][mk.cand][mk.round] += ms;
-			t.units[mk.cls][mk.cand][mk.round] += mk.units;
+			for (int q = 0; q < kNumChunks; q++) {
+				if (mk.units < (long long)kChunks[q] * kMinGroups) break;
+				if (mk.cand != 0 && mk.cand != q) continue;
+				TileTuner::Sum &u = mk.cand == 0 ? t.one[mk.cls][q][mk.round] : t.sum[mk.cls][q][mk.round];
+				u.ms += ms;
+				u.units += mk.units;
+			}
 		}
 	}
 	t.marks.clear();
 	t.used = 0;
 	if (++t.step < kTuneSteps) return;
+	const auto per_unit = [](const TileTuner::Sum *rounds) {
+		double per = -1;
+		for (int r = 0; r < 2; r++) {
+			if (rounds[r].units <= 0) continue;
+			const double v = rounds[r].ms / (double)rounds[r].units;
+			if (per < 0 || v < per) per = v;
+		}
+		return per;
+	};
 	for (int c = 0; c < TC_COUNT; c++) {
-		double best = -1;
-		for (int q = 0; q < kNumChunks; q++) {
-			double per = -1;
-			for (int r = 0; r < 2; r++) {
-				if (t.units[c][q][r] <= 0) continue;
-				const double v = t.ms[c][q][r] / (double)t.units[c][q][r];
-				if (per < 0 || v < per) per = v;
-			}
-			if (per >= 0 && (best < 0 || per < best)) { best = per; t.best[c] = kChunks[q]; }
+		double best = 1;
+		for (int q = 1; q < kNumChunks; q++) {
+			const double per = per_unit(t.sum[c][q]), one = per_unit(t.one[c][q]);
+			if (per < 0 || one <= 0 || per / one >= best) continue;
+			best = per / one;
+			t.best[c] = kChunks[q];
 		}
 	}
 	t.done = true;
