@@ -2169,15 +2169,22 @@ __host__ __device__ inline int pair_pitch(int m) { return (m + 3) & ~1; }
 __host__ __device__ inline long long pair_lds_bytes(const LevelView &L, int elem) {
 	return (long long)pair_pitch(L.m) * (L.n + 2) * (L.o + 2) * elem;
 }
-// Wavefronts of colour pair p.
-__host__ __device__ inline int pair_waves(const LevelView &L, int p) {
-	return (((L.m + 1) >> 1) * ((L.n - (p & 1) + 1) >> 1) * ((L.o - (p >> 1) + 1) >> 1) + 63) >> 6;
+// Point pairs of colour pair p.
+__host__ __device__ inline int pair_count(const LevelView &L, int p) {
+	return ((L.m + 1) >> 1) * ((L.n - (p & 1) + 1) >> 1) * ((L.o - (p >> 1) + 1) >> 1);
 }
-// Threads of the workgroup that takes level L, or 0.
+__host__ __device__ inline int pair_waves(const LevelView &L) {
+	int w = 0;
+	for (int p = 0; p < 4; p++) w += (pair_count(L, p) + 63) >> 6;
+	return w;
+}
+// Threads of the workgroup that takes level L, or 0.  A colour pair that does
+// not start at a wavefront (kept for where 12 wavefronts are too few
+// otherwise: 3x5x68) has one wavefront run its step and the next pair's.
 __host__ __device__ inline int pair_threads(const LevelView &L, int elem) {
 	if ((long long)L.m * L.n * L.o > 1024 || pair_lds_bytes(L, elem) > kSmallLdsBytes) return 0;
-	const int w = pair_waves(L, 0) + pair_waves(L, 1) + pair_waves(L, 2) + pair_waves(L, 3);
-	return w <= 8 ? 512 : w <= 12 ? 768 : 0;
+	const int w = pair_waves(L);
+	return w <= 8 ? 512 : w <= 12 || ((L.m + 1) >> 1) * L.n * L.o <= 768 ? 768 : 0;
 }
 
 template <typename T, int NT>
@@ -2196,28 +2203,27 @@ __device__ __forceinline__ void gs_lds_pairs(const LevelView &L, const T *__rest
 	long long at = 0;
 	V2 c[27], rv;
 	T ix = (T)0, iy = (T)0;
-	int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+	int it = tid, my_it = 0;
+	const bool whole = pair_waves(L) <= 12;  // colour pairs start at wavefronts
 	for (int p = 0; p < 4; p++) {
-		const int pw = pair_waves(L, p);
-		if (my < 0 && w < pw) {
-			my = p;
-			const int cj = p & 1, ck = p >> 1, nb = (L.n - cj + 1) >> 1, nd = (L.o - ck + 1) >> 1;
-			const int it = 64 * w + (tid & 63), a = it % np, b = (it / np) % nb, d = it / (np * nb);
-			if (d < nd) {
-				const int i0 = 2 * a, j = 2 * b + cj, k = 2 * d + ck;
-				live = true;
-				two = i0 + 1 < L.m;
-				lq = (i0 + 1) + hx * (j + 1) + hxy * (k + 1);
-				at = idx3(L, i0, j, k);
-				rv = *(const V2 *)(r + at);
-				const T *Ap = A + aidx3(L, 0, i0, j, k);
+		const int cnt = pair_count(L, p);
+		if (it >= 0 && it < cnt) { my = p; my_it = it; }
+		it -= whole ? (cnt + 63) & ~63 : cnt;
+	}
+	if (my >= 0) {
+		const int cj = my & 1, ck = my >> 1, nb = (L.n - cj + 1) >> 1;
+		const int a = my_it % np, b = (my_it / np) % nb, d = my_it / (np * nb);
+		const int i0 = 2 * a, j = 2 * b + cj, k = 2 * d + ck;
+		live = true;
+		two = i0 + 1 < L.m;
+		lq = (i0 + 1) + hx * (j + 1) + hxy * (k + 1);
+		at = idx3(L, i0, j, k);
+		rv = *(const V2 *)(r + at);
+		const T *Ap = A + aidx3(L, 0, i0, j, k);
 #pragma unroll
-				for (int e = 0; e < 27; e++) c[e] = *(const V2 *)(Ap + e * L.pa);
-				ix = (T)1 / c[13].x;
-				iy = (T)1 / c[13].y;
-			}
-		}
-		w -= pw;
+		for (int e = 0; e < 27; e++) c[e] = *(const V2 *)(Ap + e * L.pa);
+		ix = (T)1 / c[13].x;
+		iy = (T)1 / c[13].y;
 	}
 	__syncthreads();
 	T xe = (T)0, xd = (T)0;
@@ -2240,6 +2246,75 @@ __global__ __launch_bounds__(NT) void k_gs_pairs(LevelView L, const T *__restric
 	gs_lds_pairs<T, NT>(L, A, x, r, nsweeps, (T *)smem_);
 }
 
+// Forward colour sweeps of a non-periodic level of one point along x and at most
+// 2 NT points: two points a thread, its nine entries of the plane in registers.
+// The 18 others meet zeros of the halo, so together they are 0, or NaN where one
+// is not finite.  (One point along x leaves half of each point pair empty: 24
+// sweeps of 1x24x32 FP64 68 us by pairs, 60 by a point a thread, 32 so.)
+constexpr int kFlatThreads = 768;
+__host__ __device__ inline bool flat_ok(const LevelView &L) { return L.m == 1 && !L.prd && L.n * L.o <= 1024; }
+template <typename T, int NT>
+__device__ __forceinline__ void gs_lds_flat(const LevelView &L, const T *__restrict__ A, T *__restrict__ x,
+					    const T *__restrict__ r, int nsweeps, T *__restrict__ xs) {
+	const int tid = threadIdx.x, hy = L.n + 2, npts = L.n * L.o;
+	for (int q = tid; q < hy * (L.o + 2); q += NT) xs[q] = x[idx3(L, 0, q % hy - 1, q / hy - 1)];
+	int of[2] = {-1, -1}, lq[2];  // each point's colour class, place in LDS
+	long long at[2];
+	T c[2][9], out[2], rv[2];
+#pragma unroll
+	for (int h = 0; h < 2; h++) {
+		int q = tid + h * NT, p = 0, nb = 0;
+		if (q >= npts) continue;
+		for (; p < 4; p++) {
+			nb = (L.n - (p & 1) + 1) >> 1;
+			const int cnt = nb * ((L.o - (p >> 1) + 1) >> 1);
+			if (q < cnt) break;
+			q -= cnt;
+		}
+		const int j = 2 * (q % nb) + (p & 1), k = 2 * (q / nb) + (p >> 1);
+		of[h] = p;
+		lq[h] = (j + 1) + hy * (k + 1);
+		at[h] = idx3(L, 0, j, k);
+		rv[h] = r[at[h]];
+		const T *Ap = A + aidx3(L, 0, 0, j, k);
+		out[h] = (T)0;
+#pragma unroll
+		for (int e = 0; e < 27; e++) {
+			if (e % 3 == 1) c[h][e / 3] = Ap[e * L.pa];
+			else out[h] = out[h] + Ap[e * L.pa] * (T)0;
+		}
+		c[h][4] = (T)1 / c[h][4];
+	}
+	__syncthreads();
+#pragma unroll 1
+	for (int sw = 0; sw < nsweeps; sw++) {
+#pragma unroll 1
+		for (int p = 0; p < 4; p++) {
+			if ((p & 1) >= L.n || (p >> 1) >= L.o) continue;  // no such points
+#pragma unroll
+			for (int h = 0; h < 2; h++) {
+				if (of[h] != p) continue;
+				T ax = out[h];
+#pragma unroll
+				for (int e = 0; e < 9; e++)
+					if (e != 4) ax = ax + c[h][e] * xs[lq[h] + e % 3 - 1 + (e / 3 - 1) * hy];
+				xs[lq[h]] = (rv[h] - ax) * c[h][4];
+			}
+			__syncthreads();
+		}
+	}
+#pragma unroll
+	for (int h = 0; h < 2; h++)
+		if (of[h] >= 0) x[at[h]] = xs[lq[h]];
+}
+
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void k_gs_flat(LevelView L, const T *__restrict__ A, T *__restrict__ x,
+						const T *__restrict__ r, int nsweeps) {
+	extern __shared__ __align__(16) char smem_[];
+	gs_lds_flat<T, NT>(L, A, x, r, nsweeps, (T *)smem_);
+}
+
 template <typename T>
 __global__ __launch_bounds__(1024) void k_gs_small_lds(LevelView L, const T *__restrict__ A, T *__restrict__ x,
 						       const T *__restrict__ r, int nsweeps, int mode, int exact) {
@@ -2256,8 +2331,11 @@ __global__ __launch_bounds__(1024) void k_gs_small(LevelView L, const T *__restr
 template <typename T>
 void launch_gs_small(hipStream_t s, const LevelView &L, const T *A, T *x, const T *r, int nsweeps, int mode, int exact) {
 	const long long lds = small_lds_bytes(L, (int)sizeof(T));
-	const int nt = exact || mode || nsweeps < 1 ? 0 : pair_threads(L, (int)sizeof(T));
-	if (nt == 512)
+	const bool sweeps = !exact && !mode && nsweeps > 0;  // forward colour sweeps
+	const int nt = sweeps ? pair_threads(L, (int)sizeof(T)) : 0;
+	if (sweeps && flat_ok(L))
+		hipLaunchKernelGGL((k_gs_flat<T, kFlatThreads>), dim3(1), dim3(kFlatThreads), sizeof(T) * (L.n + 2) * (L.o + 2), s, L, A, x, r, nsweeps);
+	else if (nt == 512)
 		hipLaunchKernelGGL((k_gs_pairs<T, 512>), dim3(1), dim3(512), (unsigned)pair_lds_bytes(L, (int)sizeof(T)), s, L, A, x, r, nsweeps);
 	else if (nt == 768)
 		hipLaunchKernelGGL((k_gs_pairs<T, 768>), dim3(1), dim3(768), (unsigned)pair_lds_bytes(L, (int)sizeof(T)), s, L, A, x, r, nsweeps);
@@ -4533,8 +4611,10 @@ __global__ __launch_bounds__(256) void kb_gs_pair(const SlotDev *__restrict__ sl
 	}
 }
 
-// 768 threads: the most k_gs_pairs takes; a level with point pairs in more
-// wavefronts takes the one-point-a-thread form where it has a thread a point.
+// 768 threads: the most k_gs_pairs takes.  (The pairs of a level of one point
+// along x do not fit them from 769 points on: 16 problems of 1x30x30, 40 cycles,
+// took 12.4 ms in FP64 by a loop over the points with coefficients read again
+// each sweep; 3.0 by gs_lds_flat, 4.4 with a point a thread of 1024.)
 constexpr int kBatchSmall = 768;
 template <typename T, int NT>
 __global__ __launch_bounds__(NT) void kb_gs_tile(const SlotDev *__restrict__ slots, WorkList wl, int level, int from_zero,
@@ -4556,10 +4636,10 @@ __global__ __launch_bounds__(kBatchSmall) void kb_gs_small(const SlotDev *__rest
 	BATCH_LOOP
 		(void)lu;
 		const LevelView L = S->lv[level];
-		if (pair_threads(L, (int)sizeof(T)) > 0)
+		if (flat_ok(L))
+			gs_lds_flat<T, kBatchSmall>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), nsweeps, (T *)smem_);
+		else if (pair_threads(L, (int)sizeof(T)) > 0)
 			gs_lds_pairs<T, kBatchSmall>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), nsweeps, (T *)smem_);
-		else if (small_lds_bytes(L, (int)sizeof(T)) <= kSmallLdsBytes)
-			gs_lds_body<T>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), nsweeps, 0, 0, (T *)smem_);
 		else
 			gs_small_body<T>(L, sA<T>(S, level), sx<T>(S, level), sr<T>(S, level), nsweeps, 0, 0);
 		__syncthreads();
