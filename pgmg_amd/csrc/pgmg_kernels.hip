@@ -3710,9 +3710,21 @@ static void launch_coef_tail(hipStream_t s, const LevelView &L, double *A) {
 	HIPCHECK_LAUNCH();
 }
 
+// Coarse points below which a level with periodic axes takes k_rat_prd over all of
+// them: the interior's launch costs more than it saves.  First coarse operator,
+// all axes periodic: 16x16x16 points 80 us in one launch and 147 in two,
+// 24x20x28 182 and 182 (with the levels below 376 and 386), 32x32x32 355 and 239;
+// y periodic, 33x31x20 238 and 187.
+constexpr long long kRatPrdSplit = 1LL << 14;
+
 void launch_rat(hipStream_t s, const LevelView &F, const LevelView &C, const double *Af, double *Ac) {
 	const int lastx = (F.m - 1) >> 1, lasty = (F.n - 1) >> 1, lastz = (F.o - 1) >> 1;
-	if (lastx > 1 && lasty > 1 && lastz > 1) {
+	RatEdges E = rat_edges(F, C);
+	if (F.prd && (long long)C.m * C.n * C.o < kRatPrdSplit) {
+		E.nbx = C.m; E.nby = C.n; E.nbz = C.o;
+		E.na = (long long)C.m * C.n * C.o;
+		E.nb = E.nc = 0;
+	} else if (lastx > 1 && lasty > 1 && lastz > 1) {
 		const long long ni = (long long)(lastx - 1) * (lasty - 1) * (lastz - 1);
 		if (ni < kRatEntrySplit) {
 			const dim3 gi((unsigned)((ni + 255) / 256), 27);
@@ -3725,7 +3737,6 @@ void launch_rat(hipStream_t s, const LevelView &F, const LevelView &C, const dou
 		}
 		HIPCHECK_LAUNCH();
 	}
-	const RatEdges E = rat_edges(F, C);
 	const long long nbnd = (E.na + E.nb + E.nc) * 27;
 	const dim3 gb((unsigned)((nbnd + 255) / 256));
 	if (F.prd) hipLaunchKernelGGL(k_rat_prd, gb, dim3(256), 0, s, F, C, Af, Ac, E);
