@@ -527,18 +527,18 @@ int slot_setup(pgmg_batch *b, int s, const pgmg_dims *d, int family, uint64_t se
 		const long long N0 = (long long)D.lv[0].m * D.lv[0].n * D.lv[0].o;
 		double *stage = nullptr;
 		// and, after the operator, whether it has an entry outside the
-		// 7-point cross
+		// 7-point cross (where that matters)
 		BHIP(hipMalloc(&stage, sizeof(double) * (27 * (size_t)N0 + 1)));
-		int *dense = (int *)(stage + 27 * N0);
-		launch_fill<int>(st, dense, 1, 0);
+		int *dense = cross_pays(D.lv[0]) ? (int *)(stage + 27 * N0) : nullptr;
+		if (dense) launch_fill<int>(st, dense, 1, 0);
 		BHIP(hipMemcpyAsync(stage, A27, sizeof(double) * 27 * N0, hipMemcpyHostToDevice, st));
 		launch_pack_op(st, D.lv[0], stage, D.A[0], 0, N0, dense);
-		BHIP(hipMemcpyAsync(b->h_aux + 2 * s + 1, dense, sizeof(int), hipMemcpyDeviceToHost, st));
+		if (dense) BHIP(hipMemcpyAsync(b->h_aux + 2 * s + 1, dense, sizeof(int), hipMemcpyDeviceToHost, st));
 		BHIP(hipMemcpyAsync(stage, rhs, sizeof(double) * N0, hipMemcpyHostToDevice, st));
 		launch_pack_vec(st, D.lv[0], stage, D.r[0], 0, N0);
 		BHIP(hipStreamSynchronize(st));
 		hipFree(stage);
-		D.lv[0].cross = *(const int *)(b->h_aux + 2 * s + 1) == 0 && cross_pays(D.lv[0]);
+		D.lv[0].cross = dense && *(const int *)(b->h_aux + 2 * s + 1) == 0;
 	}
 	for (int l = 1; l < S.nl; l++) launch_rat(st, D.lv[l - 1], D.lv[l], D.A[l - 1], D.A[l]);
 	if (S.want_lu) {

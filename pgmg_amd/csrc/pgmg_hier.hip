@@ -713,19 +713,20 @@ int pgmg_level_dims(const pgmg_hier *h, int level, int dims[3]) {
 	return PGMG_OK;
 }
 
-// Host operator into level 0, and whether it is a 7-point cross (its 20 other
-// entries zero at every point), which the smoother and residual kernels use.
+// Host operator into level 0, and, where it matters, whether it is a 7-point
+// cross (its 20 other entries zero at every point), which the smoother and
+// residual kernels use.
 static int upload_op(pgmg_hier *h, const double *A27) {
 	Level &L = h->lev[0];
 	const long long N = L.points();
 	const long long chunk = 1 << 20;
 	double *stage = nullptr;
-	int *dense = (int *)(h->dscalar + 2);
+	int *dense = cross_pays(L.v) ? (int *)(h->dscalar + 2) : nullptr;
 	HIP_TRY(hipMalloc(&stage, sizeof(double) * 27 * (size_t)std::min(N, chunk)));
 	// from here on the level holds neither operator: read every entry
 	L.v.cross = 0;
 	free_graphs(h);
-	launch_fill<int>(h->stream, dense, 1, 0);
+	if (dense) launch_fill<int>(h->stream, dense, 1, 0);
 	for (long long p0 = 0; p0 < N; p0 += chunk) {
 		const long long cnt = std::min(chunk, N - p0);
 		hipError_t e = hipMemcpyAsync(stage, A27 + 27 * p0, sizeof(double) * 27 * cnt, hipMemcpyHostToDevice, h->stream);
@@ -734,11 +735,12 @@ static int upload_op(pgmg_hier *h, const double *A27) {
 		hipStreamSynchronize(h->stream);
 	}
 	hipFree(stage);
+	if (!dense) return PGMG_OK;
 	HIP_TRY(hipMemcpyAsync(h->hscalar + 2, h->dscalar + 2, sizeof(double), hipMemcpyDeviceToHost, h->stream));
 	HIP_TRY(hipStreamSynchronize(h->stream));
 	int d = 1;
 	memcpy(&d, h->hscalar + 2, sizeof(int));
-	L.v.cross = d == 0 && cross_pays(L.v);
+	L.v.cross = d == 0;
 	return PGMG_OK;
 }
 
