@@ -71,6 +71,12 @@ int pgmg::set_error(int code, const char *msg) {
 	return code;
 }
 
+// Vectors of up to this many bytes are read out through memory that a hierarchy
+// pins anyway: a program that makes a hierarchy for one small system pays for no
+// buffer on its read-out (9^3, first read-out 28 us with a buffer of its own, 16
+// so).
+const size_t kSmallReadout = 16 << 10;
+
 struct pgmg_hier {
 	int device = 0;
 	hipStream_t stream = nullptr;
@@ -86,8 +92,9 @@ struct pgmg_hier {
 	                            // sweeps' wait flag (set when a wait gave up),
 	                            // that in the third the upload's dense-operator
 	                            // flag
-	double *hscalar = nullptr;  // pinned: a reduction's result, and the mirror
-	                            // of the two flags
+	double *hscalar = nullptr;  // pinned: a reduction's result, the mirror of
+	                            // the two flags, and 64 bytes on a read-out
+	                            // buffer of kSmallReadout bytes
 	int *flow_prog = nullptr;   // plane progress counters of the exact sweeps
 	int flow_limit = kFlowLimit;
 	double *LU = nullptr;
@@ -671,7 +678,8 @@ int pgmg_hier_create(const pgmg_dims *d, const pgmg_opts *opts, pgmg_hier **out)
 	}
 	ALLOC(h->dscalar, 24);
 	launch_fill<double>(h->stream, h->dscalar, 3, 0.0);
-	if (hipHostMalloc((void **)&h->hscalar, 24) != hipSuccess) { pgmg_hier_destroy(h); return fail(PGMG_ERR_MEMORY, "pinned alloc failed"); }
+	if (hipHostMalloc((void **)&h->hscalar, 64 + kSmallReadout) != hipSuccess) { pgmg_hier_destroy(h); return fail(PGMG_ERR_MEMORY, "pinned alloc failed"); }
+	h->readout.lend(h->hscalar + 8, kSmallReadout);
 	rc = ensure_partial(h, residual_partial_count(h->lev[0].v));
 	if (rc) { pgmg_hier_destroy(h); return rc; }
 #undef ALLOC

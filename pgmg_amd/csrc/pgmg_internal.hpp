@@ -395,11 +395,14 @@ public:
 	~HostReadout();
 	// The grid points of d to out; out is complete on return.
 	hipError_t copy(hipStream_t s, const LevelView &L, const double *d, double *out);
-	static const int kSlots = 8;
+	// A pinned buffer of the owner's, for vectors that fit it until a larger
+	// one comes; before the first copy.
+	void lend(double *p, size_t bytes) { buf = p; cap = bytes; }
+	static constexpr int kSlots = 8;
 
 private:
 	std::mutex mu;
-	double *buf = nullptr;
+	double *buf = nullptr, *own = nullptr;  // own: allocated here
 	size_t cap = 0;
 	hipEvent_t ev[kSlots] = {};
 };

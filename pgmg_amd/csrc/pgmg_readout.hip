@@ -26,7 +26,7 @@ struct Feed {
 }  // namespace
 
 HostReadout::~HostReadout() {
-	if (buf) hipHostFree(buf);
+	if (own) hipHostFree(own);
 	for (auto e : ev)
 		if (e) hipEventDestroy(e);
 }
@@ -50,11 +50,12 @@ hipError_t HostReadout::copy(hipStream_t s, const LevelView &L, const double *d,
 	const size_t need = sizeof(double) * (size_t)std::min(N, slots * kChunk);
 	hipError_t e = hipSuccess;
 	if (need > cap) {
-		if (buf) hipHostFree(buf);
-		buf = nullptr;
+		if (own) hipHostFree(own);
+		own = buf = nullptr;
 		cap = 0;
-		e = hipHostMalloc((void **)&buf, need, hipHostMallocDefault);
-		if (e != hipSuccess) return e;
+		e = hipHostMalloc((void **)&own, need, hipHostMallocDefault);
+		if (e != hipSuccess) { own = nullptr; return e; }
+		buf = own;
 		cap = need;
 	}
 	for (int q = 0; q < slots; q++)

@@ -1,6 +1,7 @@
 """Calls of very small systems, whose time is launches, waits and allocations:
-an operator's upload takes no work that only larger levels have a use for, held
-against a call of the same hierarchy that does as much."""
+an operator's upload takes no work that only larger levels have a use for, and
+a new hierarchy's first read-out allocates nothing.  Each against a call of the
+same hierarchy that does as much."""
 import time
 
 import numpy as np
@@ -28,3 +29,14 @@ def test_operator_upload():
         # the same transfer, packing and wait, and the launch of the tail copies
         assert op < 2.35 * rhs
 
+
+def test_first_readout():
+    first, second = [], []
+    print("start", flush=True)
+    for _ in range(30):
+        with P.Hierarchy(9, 9, 9) as h:
+            h.synchronize()
+            first.append(timed(h.get_x))
+            second.append(timed(h.get_x))
+    print("first %.1f us, second %.1f us" % (1e6 * np.median(first), 1e6 * np.median(second)), flush=True)
+    assert np.median(first) < 1.6 * np.median(second)
