@@ -3748,20 +3748,24 @@ void launch_rat(hipStream_t s, const LevelView &F, const LevelView &C, const dou
 // ---------------------------------------------------------- bottom LU
 
 // Dense column-major matrix of the bottom level, row = point, column =
-// neighbour (region_tr.cc:486-504): entry t of the N * 27.  LU is zero before.
-__device__ __forceinline__ void lu_assemble_entry(const LevelView &L, const double *__restrict__ A, double *__restrict__ LU,
-						  long long t) {
+// neighbour (region_tr.cc:486-504): entry t of the N * 27 and its place, false
+// where the neighbour is outside the grid.
+__device__ __forceinline__ bool lu_entry(const LevelView &L, const double *__restrict__ A, long long t, double &v, long long &at) {
 	const int N = L.m * L.n * L.o;
 	const int e = (int)(t % 27), p = (int)(t / 27);
 	const int i = p % L.m, j = (p / L.m) % L.n, k = p / (L.m * L.n);
 	const int qi = i + e % 3 - 1, qj = j + (e / 3) % 3 - 1, qk = k + e / 9 - 1;
-	if (qi < 0 || qi >= L.m || qj < 0 || qj >= L.n || qk < 0 || qk >= L.o) return;
-	const int q = qi + L.m * (qj + L.n * qk);
-	LU[p + (long long)q * N] = A[aidx3(L, e, i, j, k)];
+	if (qi < 0 || qi >= L.m || qj < 0 || qj >= L.n || qk < 0 || qk >= L.o) return false;
+	v = A[aidx3(L, e, i, j, k)];
+	at = p + (long long)(qi + L.m * (qj + L.n * qk)) * N;
+	return true;
 }
+// The caller zero-fills LU first.
 __global__ void k_lu_assemble(LevelView L, const double *__restrict__ A, double *__restrict__ LU) {
 	const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (t < (long long)L.m * L.n * L.o * 27) lu_assemble_entry(L, A, LU, t);
+	double v;
+	long long at;
+	if (t < (long long)L.m * L.n * L.o * 27 && lu_entry(L, A, t, v, at)) LU[at] = v;
 }
 
 // With periodic axes, one thread per row: a wrapped neighbour's column is its
@@ -3811,18 +3815,14 @@ __host__ __device__ inline int lu_band(const LevelView &L, int N) {
 // Only the operator's band is worked on (half width `band`; N: none): column
 // c has nothing below row c + band, whatever was interchanged before, and
 // with interchanges row c ends at column c + 2 band; what is left out are
-// updates by 0.  (L's zeros below the band still take the pivot's sign.)  A
-// wavefront updates four columns at a time, a lane a row.  11x7x9 unknowns:
-// 33 ms over the whole matrix with one entry a thread and a 64-bit division for
-// each, 5.1 so.  The largest entry is found with one barrier: within each
-// wavefront, then by every wavefront from the 16 that remain.
-//
-// Returns whether this thread met an entry that is not finite: 0 times that is
-// NaN, so what was left out is not 0 then.
-__device__ __forceinline__ bool lu_factor_pass(int N, int band, double *__restrict__ LU, int *__restrict__ ipiv, int &s_info) {
+// updates by 0.  A wavefront updates four columns at a time, a lane a row.
+// 11x7x9 unknowns: 33 ms over the whole matrix with one entry a thread and a
+// 64-bit division for each, 5.3 so.  The largest entry is found with one
+// barrier: within each wavefront, then by every wavefront from the ones (a power
+// of two of them) that remain.
+__device__ __forceinline__ void lu_factor_pass(int N, int band, double *__restrict__ LU, int *__restrict__ ipiv, int &s_info) {
 	__shared__ double bv[16];
 	__shared__ int bi[16];
-	bool odd = false;
 	const int tid = threadIdx.x, nt = blockDim.x;
 	const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	if (tid == 0) s_info = 0;
@@ -3843,8 +3843,8 @@ __device__ __forceinline__ bool lu_factor_pass(int N, int band, double *__restri
 		for (int w = 32; w > 0; w >>= 1) better(__shfl_xor(best, w, 64), __shfl_xor(at, w, 64), best, at);
 		if (lane == 0) { bv[wave] = best; bi[wave] = at; }
 		__syncthreads();
-		best = bv[lane & 15];
-		at = bi[lane & 15];
+		best = bv[lane & (nt / 64 - 1)];
+		at = bi[lane & (nt / 64 - 1)];
 		for (int w = 8; w > 0; w >>= 1) better(__shfl_xor(best, w, 64), __shfl_xor(at, w, 64), best, at);
 		// The sequential rule keeps the diagonal unless another entry is
 		// strictly larger; a NaN column keeps the diagonal.  Every thread
@@ -3867,11 +3867,7 @@ __device__ __forceinline__ bool lu_factor_pass(int N, int band, double *__restri
 				__syncthreads();
 			}
 			const double rp = 1.0 / pivot;
-			for (int r = c + 1 + tid; r < N; r += nt) {
-				const double l = Lc[r] * rp;
-				Lc[r] = l;
-				odd |= !(fabs(l) <= kLargest);
-			}
+			for (int r = c + 1 + tid; r < rend; r += nt) Lc[r] *= rp;
 		} else if (tid == 0 && s_info == 0) {
 			s_info = c + 1;
 		}
@@ -3880,10 +3876,7 @@ __device__ __forceinline__ bool lu_factor_pass(int N, int band, double *__restri
 		for (int j0 = c + 1 + 4 * wave; j0 < cend; j0 += 4 * (nt / 64)) {
 			double u[4];
 #pragma unroll
-			for (int q = 0; q < 4; q++) {
-				u[q] = j0 + q < cend ? LU[(long long)(j0 + q) * N + c] : 0.0;
-				odd |= !(fabs(u[q]) <= kLargest);
-			}
+			for (int q = 0; q < 4; q++) u[q] = j0 + q < cend ? LU[(long long)(j0 + q) * N + c] : 0.0;
 			for (int r = c + 1 + lane; r < rend; r += 64) {
 				const double l = Lc[r];
 				double v[4];
@@ -3896,24 +3889,50 @@ __device__ __forceinline__ bool lu_factor_pass(int N, int band, double *__restri
 		}
 		__syncthreads();
 	}
+}
+
+// What a pass over the band leaves to do: L's zeros below the band take their
+// pivot's sign.  Returns whether this thread met an entry that is not finite: 0
+// times that is NaN, so what was left out is not 0 then.
+__device__ __forceinline__ bool lu_factor_check(int N, double *__restrict__ LU) {
+	bool odd = false;
+	for (int c = threadIdx.x >> 6; c < N; c += blockDim.x >> 6) {
+		double *const Lc = LU + (long long)c * N;
+		const bool negative = Lc[c] < 0.0;
+#pragma unroll 8
+		for (int r = threadIdx.x & 63; r < N; r += 64) {
+			const double v = Lc[r];
+			odd |= !(fabs(v) <= kLargest);
+			if (negative && r > c && v == 0.0) Lc[r] = -0.0;
+		}
+	}
 	return odd;
 }
 
-// A factor in which the band met an infinity or a NaN is made again, from the
-// operator, over the whole matrix, where such an entry reaches rows below the
-// band (11x7x9 unknowns 24.7 ms, 5.4 without).
+// An operator with an infinity or a NaN is factored over the whole matrix, where
+// such an entry reaches rows below the band; one whose band comes to such an
+// entry on the way is factored again (11x7x9 unknowns 5.3 ms, whole 19.3).
 __global__ __launch_bounds__(1024) void k_lu_factor(LevelView L, const double *__restrict__ A, int N,
 						    double *__restrict__ LU, int *__restrict__ ipiv, int *__restrict__ info) {
 	__shared__ int s_info;
 	const int tid = threadIdx.x, nt = blockDim.x;
-	for (int band = lu_band(L, N);;) {
-		const bool odd = lu_factor_pass(N, band, LU, ipiv, s_info);
-		if (!__syncthreads_or(odd) || band >= N) break;
+	double v;
+	long long at;
+	int band = lu_band(L, N), odd = 0;
+	if (band < N) {
+		for (long long t = tid; t < 27LL * N; t += nt)
+			if (lu_entry(L, A, t, v, at)) odd |= !(fabs(v) <= kLargest);
+		if (__syncthreads_or(odd)) band = N;
+	}
+	lu_factor_pass(N, band, LU, ipiv, s_info);
+	odd = band < N && lu_factor_check(N, LU);
+	if (__syncthreads_or(odd)) {
 		for (long long q = tid; q < (long long)N * N; q += nt) LU[q] = 0.0;
 		__syncthreads();
-		for (long long t = tid; t < 27LL * N; t += nt) lu_assemble_entry(L, A, LU, t);
+		for (long long t = tid; t < 27LL * N; t += nt)
+			if (lu_entry(L, A, t, v, at)) LU[at] = v;
 		__syncthreads();
-		band = N;
+		lu_factor_pass(N, N, LU, ipiv, s_info);
 	}
 	if (tid == 0) {
 		info[0] = s_info;
@@ -3923,7 +3942,11 @@ __global__ __launch_bounds__(1024) void k_lu_factor(LevelView L, const double *_
 }
 
 void launch_lu_factor(hipStream_t s, const LevelView &L, const double *A, double *LU, int *ipiv, int *info) {
-	hipLaunchKernelGGL(k_lu_factor, dim3(1), dim3(1024), 0, s, L, A, L.m * L.n * L.o, LU, ipiv, info);
+	const int N = L.m * L.n * L.o;
+	// few unknowns are bound by the barriers, which cost less among 8 wavefronts:
+	// 27 unknowns 97 us (16 wavefronts 110), 125 434 (464), 216 870 (869), 693
+	// 5.8 ms (5.3)
+	hipLaunchKernelGGL(k_lu_factor, dim3(1), dim3(N <= 200 ? 512 : 1024), 0, s, L, A, N, LU, ipiv, info);
 	HIPCHECK_LAUNCH();
 }
 
