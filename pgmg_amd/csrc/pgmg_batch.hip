@@ -236,12 +236,27 @@ void plan_add(pgmg_batch *b, int li, int slot, int units) {
 // 256, 483 with 512, 453 with 1024, 498 with 1536 and more.
 const long long kMaxTiles = 1024;
 
+// Level-0 coefficients that the 7-point slots' lists of their own save a sweep,
+// from which they are kept where other slots are active too: below, the second
+// set of launches costs more.  Joined and split lists, 25 cycles, 65^3 unless
+// said: one 7-point and one 27-point problem FP64 (44 MB) 13.8 and 14.8 ms, two
+// and two (88 MB) 20.2 and 20.9, 97^3 one and one (146 MB) 31.2 and 30.3, four
+// and one (176 MB) 22.0 and 19.0; FP32 two and two (44 MB) 14.0 and 15.7, four
+// and four (88 MB) 23.7 and 24.0, two of 97^3 and a 40^3 (146 MB) 26.4 and 22.2.
+const long long kCrossBytes = 96LL << 20;
+
 int build_plan(pgmg_batch *b) {
 	const int el = b->mixed ? 4 : 8;  // the cycle's arithmetic
-	long long tiles[kBatchMaxLevels] = {};
+	long long tiles[kBatchMaxLevels] = {}, saved = 0;
+	bool dense = false;
 	for (const SlotHost &S : b->slots)
-		if (S.state == ST_ACTIVE)
+		if (S.state == ST_ACTIVE) {
+			const LevelView &L = S.dev.lv[0];
 			for (int l = 0; l < S.nl; l++) tiles[l] += S.tiles[l];
+			if (L.cross) saved += 20LL * el * L.m * L.n * L.o;
+			else dense = true;
+		}
+	const bool split = !dense || saved >= kCrossBytes;
 	memset(b->tile_lds, 0, sizeof b->tile_lds);
 	std::fill(b->list_n.begin(), b->list_n.end(), 0);
 	b->level_bytes.assign(kBatchMaxLevels, 0);
@@ -252,12 +267,12 @@ int build_plan(pgmg_batch *b) {
 		if (S.state != ST_ACTIVE) continue;
 		const SlotDev &D = S.dev;
 		b->max_nl = std::max(b->max_nl, S.nl);
-		plan_add(b, D.lv[0].cross ? L_X_TOP_ROWS : L_TOP_ROWS, s, batch_units(BK_ROWS, D.lv[0], 8));
+		plan_add(b, split && D.lv[0].cross ? L_X_TOP_ROWS : L_TOP_ROWS, s, batch_units(BK_ROWS, D.lv[0], 8));
 		plan_add(b, L_TOP_ONE, s, 1);
 		plan_add(b, L_TOP_PTS, s, batch_units(BK_FLAT, D.lv[0], 8));
 		for (int l = 0; l < S.nl; l++) {
 			const LevelView &L = D.lv[l];
-			const bool x = L.cross != 0;  // level 0 only
+			const bool x = split && L.cross;  // level 0 only
 			b->level_bytes[l] += (x ? 7LL : 27LL) * el * L.m * L.n * L.o;
 			if (l < S.nl - 1) {
 				// as the lone hierarchy's forward colour sweeps
