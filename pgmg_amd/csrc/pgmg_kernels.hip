@@ -2181,8 +2181,11 @@ __host__ __device__ inline int pair_waves(const LevelView &L) {
 // Threads of the workgroup that takes level L, or 0.  A colour pair that does
 // not start at a wavefront (kept for where 12 wavefronts are too few
 // otherwise: 3x5x68) has one wavefront run its step and the next pair's.
+// Not for one point along x, where half of each pair is empty: gs_lds_flat, or
+// with periodic axes a point a thread (24 sweeps of 1x154x4, y and z periodic, FP64
+// 118 us by pairs, 98 so).
 __host__ __device__ inline int pair_threads(const LevelView &L, int elem) {
-	if ((long long)L.m * L.n * L.o > 1024 || pair_lds_bytes(L, elem) > kSmallLdsBytes) return 0;
+	if (L.m == 1 || (long long)L.m * L.n * L.o > 1024 || pair_lds_bytes(L, elem) > kSmallLdsBytes) return 0;
 	const int w = pair_waves(L);
 	return w <= 8 ? 512 : w <= 12 || ((L.m + 1) >> 1) * L.n * L.o <= 768 ? 768 : 0;
 }

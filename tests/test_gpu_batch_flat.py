@@ -35,19 +35,19 @@ def same_bits(a, b):
     return np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(a[~np.isnan(a)], b[~np.isnan(b)])
 
 
-@pytest.mark.parametrize("shape", SHAPES)
-def test_sweeps_bitwise(shape):
+@pytest.mark.parametrize("shape,prd", [(s, 0) for s in SHAPES] + [((1, 154, 4), 6), ((1, 30, 30), 7), ((1, 9, 8), 1), ((1, 1, 700), 4)])
+def test_sweeps_bitwise(shape, prd):
     m, n, o = shape
-    print("case", shape, flush=True)
-    A, b = O.gen_operator(P.FAM_Q1_ANISO, 5, m, n, o), O.gen_rhs(5, m, n, o)
+    print("case", shape, prd, flush=True)
+    A, b = O.gen_operator(P.FAM_Q1_ANISO, 5, m, n, o, prd=prd), O.gen_rhs(5, m, n, o)
     x = O.test_field(m, n, o, 3)
     x[o // 2, n // 2, m // 2] = np.inf
-    with P.Hierarchy(m, n, o) as h:
+    with P.Hierarchy(m, n, o, prd=prd) as h:
         h.set_operator27(A)
         h.set_rhs(b)
         h.set_x(x)
         h.gauss_seidel(0, 0, 2)
-        mg = O.Multigrid(A, colour8=True)
+        mg = O.Multigrid(A, colour8=True, prd=prd)
         mg.set_rhs(b)
         mg.set_x(0, x)
         for _ in range(2):
@@ -72,6 +72,27 @@ def test_batch_entry_outside_the_plane():
             h.solve(1e-8, 3)
         assert np.isnan(h.get_x()).any()
         assert same_bits(batch.get_x(s), h.get_x())
+
+
+def sweeps_time(shape, prd):
+    best = 1e9
+    with P.Hierarchy(*shape, prd=prd) as h:
+        h.generate_problem(P.FAM_Q1_ANISO, 5)
+        for _ in range(6):
+            t = time.perf_counter()
+            for _ in range(10):
+                h.gauss_seidel(0, 0, 24)
+            h.synchronize()
+            best = min(best, (time.perf_counter() - t) / 10)
+    return 1e6 * best
+
+
+def test_periodic_sweeps_time():
+    # 616 points, of one and of two along x, ghosts refreshed in each sweep
+    print("start", flush=True)
+    one, two = sweeps_time((1, 154, 4), 6), sweeps_time((2, 77, 4), 6)
+    print("24 sweeps: 1x154x4 %.1f us, 2x77x4 %.1f us" % (one, two), flush=True)
+    assert one < 1.05 * two
 
 
 def batch_time(shape, precision):
