@@ -2183,9 +2183,13 @@ __host__ __device__ inline int pair_waves(const LevelView &L) {
 // otherwise: 3x5x68) has one wavefront run its step and the next pair's.
 // Not for one point along x, where half of each pair is empty: gs_lds_flat, or
 // with periodic axes a point a thread (24 sweeps of 1x154x4, y and z periodic, FP64
-// 118 us by pairs, 98 so).
+// 118 us by pairs, 98 so).  Nor for periodic planes and lines, which have more
+// threads to refresh the ghosts so and no use for half of the steps: 244x1x2, y
+// and z periodic, 134 us by pairs, 111 so; 169x6x1 146 and 130; 20x1x13, y
+// periodic, 62 both ways.
 __host__ __device__ inline int pair_threads(const LevelView &L, int elem) {
-	if (L.m == 1 || (long long)L.m * L.n * L.o > 1024 || pair_lds_bytes(L, elem) > kSmallLdsBytes) return 0;
+	if (L.m == 1 || (L.prd && (L.n == 1 || L.o == 1))) return 0;
+	if ((long long)L.m * L.n * L.o > 1024 || pair_lds_bytes(L, elem) > kSmallLdsBytes) return 0;
 	const int w = pair_waves(L);
 	return w <= 8 ? 512 : w <= 12 || ((L.m + 1) >> 1) * L.n * L.o <= 768 ? 768 : 0;
 }

@@ -35,7 +35,8 @@ def same_bits(a, b):
     return np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(a[~np.isnan(a)], b[~np.isnan(b)])
 
 
-@pytest.mark.parametrize("shape,prd", [(s, 0) for s in SHAPES] + [((1, 154, 4), 6), ((1, 30, 30), 7), ((1, 9, 8), 1), ((1, 1, 700), 4)])
+@pytest.mark.parametrize("shape,prd", [(s, 0) for s in SHAPES] + [((1, 154, 4), 6), ((1, 30, 30), 7), ((1, 9, 8), 1), ((1, 1, 700), 4),
+                                                         ((244, 1, 2), 6), ((169, 6, 1), 6), ((20, 1, 13), 2)])
 def test_sweeps_bitwise(shape, prd):
     m, n, o = shape
     print("case", shape, prd, flush=True)
@@ -93,6 +94,14 @@ def test_periodic_sweeps_time():
     one, two = sweeps_time((1, 154, 4), 6), sweeps_time((2, 77, 4), 6)
     print("24 sweeps: 1x154x4 %.1f us, 2x77x4 %.1f us" % (one, two), flush=True)
     assert one < 1.05 * two
+
+
+def test_periodic_plane_sweeps_time():
+    # 488 points, one plane and two
+    print("start", flush=True)
+    one, two = sweeps_time((244, 1, 2), 6), sweeps_time((122, 2, 2), 6)
+    print("24 sweeps: 244x1x2 %.1f us, 122x2x2 %.1f us" % (one, two), flush=True)
+    assert one < 1.15 * two
 
 
 def batch_time(shape, precision):
