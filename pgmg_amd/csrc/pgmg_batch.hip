@@ -201,9 +201,11 @@ void drop_graph(pgmg_batch *b) {
 // with plain loads, to find them in the memory-side cache (256 MB) in the next
 // sweep; larger levels are streamed, as when side by side they would push
 // each other out.  (A small level of a few slots streamed from HBM takes
-// twice as long a launch.)  16 problems of 33 to 129 points an axis: 857 ms
-// all streamed, 747 with 32 MB, 736 with 64, 722 with 128 and 256, 732 with
-// everything cached.
+// twice as long a launch.)  Problems of 33 to 129 points an axis, 16 in mixed
+// precision (level 0 127 MB of 7-point coefficients): 475 ms all streamed, 474
+// with 32 MB, 459 with 64, 444 with 128 and more; 16 in FP64 (253 MB) 607, 605,
+// 605, 594, and 584 with 192 and more; 32 mixed (331 MB) 968, 917, 916, 914, 889;
+// 8 mixed (52 MB) 385, 344, 331 and no less.
 const long long kCacheBytes = 128LL << 20;
 
 int list_index(int level, int kind) { return L_TOP_COUNT + level * L_PER_LEVEL + kind; }
