@@ -538,7 +538,10 @@ def main():
     tf = os.path.join(ROOT, "profiles", "traffic_gs_pair_f32_257.json")
     if os.path.exists(tf):
         try:
-            traffic = json.load(open(tf)).get("hbm_bytes_per_launch")
+            rec = json.load(open(tf))
+            # of the kernel that is timed here, or none
+            if rec["kernel"].startswith("k_gs_pair<float, false, true>"):
+                traffic = rec["hbm_bytes_per_launch"]
         except Exception:
             traffic = None
 
