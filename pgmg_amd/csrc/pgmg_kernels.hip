@@ -208,9 +208,8 @@ template <> __device__ __forceinline__ double2 ld_stream<double2>(const void *ba
 // (0 * x), so the sums are those of the 27 planes for every x, infinities and
 // NaN included; e must be a compile-time constant after unrolling.  The row
 // kernels are bound by HBM bytes, and 20 of the 27 planes of a 7-point
-// operator hold only zeros: 257^3 level-0 smoother launch FP32 98 -> 42 us
-// (5.3 TB/s of the 13 words a point it then moves), FP64 210 -> 101 us; FP64
-// residual 666 -> 301 us.
+// operator hold only zeros: 257^3 level-0 smoother launch FP32 98 -> 40.5 us
+// (580 -> 242 MB, 6.0 TB/s), FP64 210 -> 96 us; FP64 residual 666 -> 286 us.
 template <typename V, bool X, typename T>
 __device__ __forceinline__ V coef_or_zero(const T *Ar, int e, long long pa, uint32_t off) {
 	if (X && !in_cross(e)) {
