@@ -11,7 +11,10 @@
  *
  * One hierarchy lives on one GPU and owns one HIP stream.  Calls on one
  * handle must come from one thread at a time; distinct handles are
- * independent.
+ * independent.  gauss_seidel, restriction, interpolation, solve_exact and
+ * v_cycle queue their work on that stream and return; the calls that take or
+ * give data, set-ups, norms, solves, pgmg_clear_x and pgmg_synchronize return
+ * when what was queued before them is complete, and report its errors.
  *
  * Layout of host arrays: point-major, p = i + m*(j + n*k).  Operators carry
  * 27 entries per point, e = (dk+1)*9 + (dj+1)*3 + (di+1): the reference's box

@@ -988,8 +988,8 @@ __device__ __forceinline__ void gs_wave(const LevelView &L, const T *__restrict_
 // (i0, i0+1), i0 = s0 + 2l; an even point's new odd neighbours are the lane's
 // own and the lane before's (shuffle; lane 0's is handed over by the segment
 // before, which is complete by then: an odd point reads only old even
-// points).  Next to the grid x is the halo's, zero or ghosts, as memory holds
-// it.  Arithmetic and order as in gs_point.
+// points).  Next to the grid x is the halo's, as memory holds it (periodic levels
+// take k_gs_colour).  Arithmetic and order as in gs_point.
 //
 // Bound by bytes: one launch a class read every line of the coefficients
 // twice, half of it each time.  161x130x147 FP64, 27 points: 86 us for two

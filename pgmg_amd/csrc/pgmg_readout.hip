@@ -37,11 +37,11 @@ HostReadout::~HostReadout() {
 // not the bus, bounds one thread (10 GB/s), and one chunk of each of up to 8
 // threads is under way at a time.  Vectors of at most four chunks are copied
 // by the caller: threads cost more than they save there.
-// Into a new array: 257^3 (136 MB) 13.7 ms by hipMemcpy from a device copy, 3.6
-// so; 161x130x147 (25 MB) 1.87 and 1.13; 33^3 57 and 39 us.  Chunks of 0.5 MB:
-// 4.4 ms, of 2 MB: 3.8.  Eight chunks: 257^3 takes 3.8 ms where 16 take 3.6, but
-// the buffer is pinned on a hierarchy's first read-out, which with 16 costs a
-// 161x130x147 program 0.3 ms more.
+// Into a new array: 257^3 (136 MB) 13.7 ms by hipMemcpy from a device copy, 3.8
+// so; 161x130x147 (25 MB) 1.87 and 1.13; 33^3 57 and 39 us.  With 16 chunks 257^3
+// takes 3.6 ms (then chunks of 0.5 MB: 4.4, of 2 MB: 3.8), but the buffer is pinned
+// on a hierarchy's first read-out, which with 16 costs a 161x130x147 program
+// 0.3 ms more.
 hipError_t HostReadout::copy(hipStream_t s, const LevelView &L, const double *d, double *out) {
 	std::lock_guard<std::mutex> one(mu);
 	const long long N = (long long)L.m * L.n * L.o;
