@@ -3975,7 +3975,7 @@ void launch_lu_factor(hipStream_t s, const LevelView &L, const double *A, double
 // are not read.  With interchanges U's upper half width is at most 2 bw and L
 // is taken as full; so are both with periodic axes.
 //
-// 11x7x9 unknowns: 675 us a solve with a barrier a column, 107 us so (122 with
+// 11x7x9 unknowns: 475 us a solve with a barrier a column, 103 us so (122 with
 // four wavefronts of twice the registers).
 const int kLuWaves = 8;
 const int kLuMax = 2048;  // enable_exact takes fewer points than this
@@ -4177,8 +4177,8 @@ __device__ __forceinline__ void lu_solve_pieces(const LevelView &L, int N, const
 // the second kind where the source does not.
 //
 // R rows a thread, in registers, with the next column's entries of them in
-// flight, one barrier a column: 11x7x9 unknowns 372 us, 4x4x4 25 (by pieces 109
-// and 14; rows in LDS, as every source was solved before the pieces, 475 and 43).
+// flight, one barrier a column: 11x7x9 unknowns 345 us, 4x4x4 24 (by pieces 103
+// and 13; rows in LDS, as every source was solved before the pieces, 475 and 43).
 template <int R>
 __device__ __forceinline__ void lu_solve_columns(int N, const double *__restrict__ LU, double *__restrict__ xs) {
 	const int nt = 64 * kLuWaves;
@@ -4242,9 +4242,11 @@ __device__ __forceinline__ void lu_solve_body(const LevelView &L, int N, const d
 		sp[q] = ipiv[q];
 		moved |= sp[q] != q;
 	}
+	// a NaN in the factor reaches its last entry, and every solution
+	const double last = LU[(long long)N * N - 1];
 	// the source into xs, interchanged; whether it is one for the columns
 	const auto load = [&] {
-		int other = 0;
+		int other = !(fabs(last) <= kLargest);
 		for (int q = tid; q < 64 * nblk; q += nt) {
 			double v = 0.0;
 			if (q < N) {
